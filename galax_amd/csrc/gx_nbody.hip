@@ -6,13 +6,15 @@
 // integrated as ONE system by OrbitSolver (shared steps; the PID error norm
 // is the RMS over all 6N state components, orbit/solver.py:121-141).
 //
-// One workgroup of 512 threads integrates the whole system (N <= 4096, the
-// range in which the reference's (N, N, 3) pair arrays are practical): the
-// stage positions of all bodies sit in LDS, every thread sums the pull of
-// all bodies on its own bodies (all lanes read the same LDS word: a
-// broadcast), stage accelerations go to a workspace in HBM, and the error
-// norm is a block reduction.  Control flow (step accept/reject, saves) is
-// uniform across the workgroup, so no host round trip happens per step.
+// One launch integrates the whole system (N <= 4096, the range in which the
+// reference's (N, N, 3) pair arrays are practical), with no host round trip
+// per step: k_nbody_grid divides the bodies among the workgroups of a
+// cooperative launch.  Where that cannot be launched (a stream capture, a
+// device partition too small), k_nbody integrates the system in one
+// workgroup of 512 threads: the stage positions of all bodies sit in LDS,
+// every thread sums the pull of all bodies on its own bodies (all lanes read
+// the same LDS word: a broadcast), stage accelerations go to a workspace in
+// HBM, and the error norm is a block reduction.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -27,6 +29,14 @@ namespace {
 
 constexpr int kNbThreads = 512;
 constexpr int kNbMax = 4096;
+// Bodies that one workgroup integrates, and fewest bodies of a workgroup when
+// there are several.  A meeting takes about 4 us whatever its size; one
+// workgroup takes that long for the pulls of 50 to 60 bodies (us a step, one
+// against several workgroups: 37 bodies 67/72, 64 bodies 73/68, 96 bodies
+// 112/69).  Workgroups of 4 bodies against 8: 1,024 bodies 103 us a step
+// against 125, 128 bodies 71 against 73 (smaller ones change nothing).
+constexpr int kNbOne = 48;
+constexpr int kNbOwnMin = 4;
 
 struct NArgs {
   double dt0, rtol, atol, safety, factormin, factormax, dtmin, dtmax;
@@ -366,6 +376,613 @@ __global__ void __launch_bounds__(kNbThreads) k_nbody(DPot P, NArgs A) {
   }
 }
 
+// ---- the system over many workgroups -------------------------------------
+// One workgroup's CU holds 1/256 of the device's FP64 rate: 1,024 bodies
+// took 600 us a stage on it (60 Myr of a cluster, 23 steps: 180.8 ms; here
+// 2.4 ms, of which the meetings take most; 128 bodies 12.3 ms, here 1.85;
+// 16 bodies, one workgroup, 4.0 ms, here 1.4).  Here the bodies are divided among G resident
+// workgroups (a cooperative launch): a workgroup owns `own` bodies, keeps
+// their state and stage accelerations in LDS, and a stage is
+//   1. the owner computes its bodies' stage positions and publishes them,
+//   2. the workgroups meet (below),
+//   3. every workgroup copies all positions to LDS, and its eight waves sum
+//      the pull on the owned bodies, lanes over the sources (a wave for a
+//      body; several waves for one when there are fewer than eight),
+//   4. the owner adds the external field, which it evaluated while waiting.
+// A meeting costs more than the sums of 1,024 bodies, so it is one store and
+// one load through the level that all XCDs share, with no flag, no
+// read-modify-write and no cache flush: every published value is its own
+// flag.  Values are written and read by relaxed device-scope atomics of 64
+// bits; a slot holds kNbEmpty (a NaN that arithmetic does not produce) until
+// its owner has published, and a reader repeats its load while it sees that.
+// Three buffers take turns by meeting.  Having read meeting k - 1, an owner
+// knows that every workgroup has come to it and so has read meeting k - 2,
+// whose buffer is the one of meeting k + 1: it empties its own slots there,
+// and waits for those stores (s_waitcnt vmcnt(0)) before it publishes for
+// meeting k, without which nobody looks at meeting k + 1.
+// Every workgroup runs the controller on the same sums in the same order
+// and takes the same decisions.  The start of a step and the end of the
+// accepted one before it are the same point, so its acceleration is kept
+// (first same as last): 13 meetings a step.
+// G = 1 is the same kernel with a workgroup barrier for a meeting and 16
+// lanes a body, for systems whose sums take less time than a meeting.
+constexpr int kNbWaves = kNbThreads / 64;
+constexpr int kNbOwnMax = 16;   // bodies of a workgroup when G > 1
+constexpr int kNbGroups = 256;  // most workgroups
+
+typedef unsigned long long NbSlot;
+constexpr NbSlot kNbEmpty = 0xfff8dead5a5a0001ull;
+constexpr NbSlot kNbNan = 0x7ff8000000000000ull;
+
+struct NGrid {
+  int G;         // workgroups
+  int own;       // bodies of a workgroup
+  NbSlot* pos;   // [3][3][n] published positions
+  NbSlot* part;  // [3][2][G] published error sums and non-finite counts
+};
+
+__global__ void k_nb_empty(NbSlot* slots, long long m) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < m) slots[i] = kNbEmpty;
+}
+
+__device__ __forceinline__ void put_slot(NbSlot* p, NbSlot v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void put_slot(NbSlot* p, double v) {
+  put_slot(p, v == v ? (NbSlot)__double_as_longlong(v) : kNbNan);
+}
+__device__ __forceinline__ NbSlot get_slot(const NbSlot* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// All G workgroups are resident and take the same decisions, so every one
+// publishes for every meeting and every wait ends.
+__device__ __forceinline__ double await_slot(const NbSlot* p, NbSlot seen) {
+  while (seen == kNbEmpty) {
+    __builtin_amdgcn_s_sleep(1);
+    seen = get_slot(p);
+  }
+  return __longlong_as_double((long long)seen);
+}
+
+// Dynamic LDS of a workgroup (doubles): all positions and masses, then the
+// owned bodies' [3][own] arrays.
+struct NbOwn {
+  double *x, *y, *z, *gm;       // [n]
+  double *q, *p, *q1, *p1;      // [3][own]
+  double *Q, *ext;              // stage position, external field
+  double* aa;                   // [S][S] the tableau squared
+  double *g;                    // [SF][3][own] stage accelerations
+  double *part;                 // [3][max(own, waves)] partial pulls
+};
+__host__ __device__ inline size_t nb_lds_doubles(long long n, int own, int SF) {
+  return (size_t)(4 * n + (long long)3 * own * (6 + SF) + 3 * (own > kNbWaves ? own : kNbWaves) +
+                  (long long)SF * SF);
+}
+
+template <class M, bool PID, class E>
+struct NbGridSolve {
+  const DPot& P;
+  const NArgs& A;
+  const NGrid& X;
+  NbOwn S;
+  double2* red;  // [waves]
+  int n, own, first, cnt, tid;
+  double dir;
+  int turn = 0;  // the buffer of the coming meeting
+
+  // Sums over the workgroup, in a fixed order; every thread gets them.
+  __device__ __forceinline__ void sum(double& a, double& b) const {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      a += __shfl_xor(a, o, 64);
+      b += __shfl_xor(b, o, 64);
+    }
+    __syncthreads();
+    if ((tid & 63) == 0) red[tid >> 6] = make_double2(a, b);
+    __syncthreads();
+    a = b = 0.0;
+#pragma unroll
+    for (int i = 0; i < kNbWaves; ++i) {
+      a += red[i].x;
+      b += red[i].y;
+    }
+  }
+
+  // Position of owned body j, component m, for the coming meeting (wave 0
+  // does all of a workgroup's publishing: own <= 16).
+  __device__ __forceinline__ void publish(int m, int j, double v) {
+    S.Q[m * own + j] = v;
+    if (X.G == 1)
+      (m == 0 ? S.x : m == 1 ? S.y : S.z)[j] = v;
+    else
+      put_slot(X.pos + ((size_t)turn * 3 + m) * n + first + j, v);
+  }
+
+  // The workgroup's two sums for the coming meeting.
+  __device__ __forceinline__ void offer(double a, double b) {
+    if (X.G == 1 || tid != 0) return;
+    NbSlot* p = X.part + (size_t)turn * 2 * X.G + blockIdx.x;
+    put_slot(p, a);
+    put_slot(p + X.G, b);
+  }
+
+  // The meeting's sums over all workgroups.
+  __device__ __forceinline__ void total(double& a, double& b) {
+    if (X.G == 1) return;
+    const NbSlot* p = X.part + (size_t)turn * 2 * X.G + tid;
+    const bool in = tid < X.G;
+    const NbSlot va = in ? get_slot(p) : 0, vb = in ? get_slot(p + X.G) : 0;
+    a = await_slot(p, va);
+    b = await_slot(p + X.G, vb);
+    sum(a, b);
+  }
+
+  // Close the meeting: empty the buffer after next, which everyone has read.
+  __device__ __forceinline__ void close() {
+    if (X.G > 1 && tid < 64) {
+      const int next = turn == 0 ? 2 : turn - 1;  // of the meeting after next
+      if (tid < 3 * cnt)
+        put_slot(X.pos + ((size_t)next * 3 + tid / cnt) * n + first + tid % cnt, kNbEmpty);
+      if (tid < 2) put_slot(X.part + ((size_t)next * 2 + tid) * X.G + blockIdx.x, kNbEmpty);
+    }
+    turn = turn == 2 ? 0 : turn + 1;
+  }
+  // Before publishing: the emptied slots have reached the shared level.
+  __device__ __forceinline__ void settle() {
+    if (X.G > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+
+  // The external field at the owned bodies' published positions.
+  __device__ __forceinline__ void external(double t) {
+    for (int j = tid; j < cnt; j += kNbThreads) {
+      double a[3];
+      E::acc(P, S.Q[j], S.Q[own + j], S.Q[2 * own + j], t, a[0], a[1], a[2]);
+      for (int m = 0; m < 3; ++m) S.ext[m * own + j] = a[m];
+    }
+  }
+
+  // All positions of the meeting into LDS.
+  __device__ __forceinline__ void fetch() {
+    if (X.G > 1) {
+      constexpr int R = 6;  // loads in flight
+      const NbSlot* src = X.pos + (size_t)turn * 3 * n;
+      for (int k0 = tid; k0 < 3 * n; k0 += R * kNbThreads) {
+        NbSlot v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int k = k0 + r * kNbThreads;
+          v[r] = k < 3 * n ? get_slot(src + k) : 0;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int k = k0 + r * kNbThreads;
+          if (k < 3 * n) S.x[k] = await_slot(src + k, v[r]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  // Pull on body `self` at (x, y, z) of the sources k0, k0 + dk, ...
+  __device__ __forceinline__ void pull(int self, double x, double y, double z, int k0, int dk,
+                                       double& ax, double& ay, double& az) const {
+    ax = ay = az = 0.0;
+#pragma unroll 8
+    for (int k = k0; k < n; k += dk) {
+      const double dx = S.x[k] - x, dy = S.y[k] - y, dz = S.z[k] - z;
+      const double r2 = dx * dx + dy * dy + dz * dz + A.eps2;
+      const double ir = rsqrt_fast(r2);
+      const double w = (k == self) ? 0.0 : S.gm[k] * ir * ir * ir;
+      ax = fma(w, dx, ax);
+      ay = fma(w, dy, ay);
+      az = fma(w, dz, az);
+    }
+  }
+
+  // Accelerations of the owned bodies at the positions in LDS, into g.
+  __device__ __forceinline__ void accelerate(double* g) {
+    const int lane = tid & 63, wave = tid >> 6;
+    int parts = 1;
+    if (X.G == 1) {
+      // 16 lanes a body, 32 bodies a round
+      for (int j0 = 0; j0 < own; j0 += kNbThreads / 16) {
+        const int j = j0 + (tid >> 4), c = j < own ? j : own - 1;
+        double ax, ay, az;
+        pull(c, S.Q[c], S.Q[own + c], S.Q[2 * own + c], tid & 15, 16, ax, ay, az);
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) {
+          ax += __shfl_xor(ax, o, 64);
+          ay += __shfl_xor(ay, o, 64);
+          az += __shfl_xor(az, o, 64);
+        }
+        if ((tid & 15) == 0 && j < own) {
+          S.part[j] = ax;
+          S.part[own + j] = ay;
+          S.part[2 * own + j] = az;
+        }
+      }
+    } else {
+      // a wave for a body, or `parts` waves when that leaves waves idle
+      while (2 * own * parts <= kNbWaves) parts *= 2;
+      for (int u = wave; u < own * parts; u += kNbWaves) {
+        const int j = u / parts, c = j < cnt ? j : 0;
+        double ax, ay, az;
+        pull(first + c, S.Q[c], S.Q[own + c], S.Q[2 * own + c], (u % parts) * 64 + lane, 64 * parts, ax, ay,
+             az);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+          ax += __shfl_xor(ax, o, 64);
+          ay += __shfl_xor(ay, o, 64);
+          az += __shfl_xor(az, o, 64);
+        }
+        if (lane == 0) {
+          S.part[u] = ax;
+          S.part[own * parts + u] = ay;
+          S.part[2 * own * parts + u] = az;
+        }
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < 3 * own; i += kNbThreads) {
+      const int m = i / own, j = i - m * own;
+      double a = S.ext[i];
+      for (int k = 0; k < parts; ++k) a += S.part[(m * own + j) * parts + k];
+      g[i] = a;
+    }
+    __syncthreads();
+  }
+
+  __device__ __forceinline__ void save(int s, const double* q, const double* p) const {
+    for (int i = tid; i < 3 * own; i += kNbThreads) {
+      const int m = i / own, j = i - m * own;
+      if (j >= cnt) continue;
+      double* o = A.out + ((size_t)(first + j) * A.T + s) * 6 + m;
+      o[0] = q[i];
+      o[3] = dir * p[i];
+    }
+  }
+
+  // A save inside the step: the method's dense output at th of it.
+  __device__ __forceinline__ void save_inside(int s, double th, double h) const {
+    constexpr int SF = M::SF;
+    double wq[SF], wp[SF];
+    dense_weights<M>(th, wq, wp);
+    const double ht = h * th, hht = h * ht;
+    for (int k = tid; k < 3 * own; k += kNbThreads) {
+      const int m = k / own, j = k - m * own;
+      if (j >= cnt) continue;
+      double a = 0.0, b = 0.0;
+#pragma unroll
+      for (int l = 0; l < SF; ++l) {
+        const double gl = S.g[l * 3 * own + k];
+        a = fma(wq[l], gl, a);
+        b = fma(wp[l], gl, b);
+      }
+      double* o = A.out + ((size_t)(first + j) * A.T + s) * 6 + m;
+      o[0] = fma(hht, a, fma(ht, S.p[k], S.q[k]));
+      o[3] = dir * fma(ht, b, S.p[k]);
+    }
+  }
+
+  __device__ __forceinline__ void run() {
+    constexpr auto& K = M::k;
+    constexpr int SF = M::SF;
+    const int own3 = 3 * own;
+    double* const gend = S.g + (SF - 1) * own3;
+    dir = (A.t0 < A.t1) ? 1.0 : -1.0;
+    for (int k = tid; k < n; k += kNbThreads) S.gm[k] = A.gm[k];
+    for (int k = tid; k < M::S * M::S; k += kNbThreads) S.aa[k] = K.aa[k / M::S][k % M::S];
+    for (int k = tid; k < SF * own3; k += kNbThreads) S.g[k] = 0.0;
+    for (int i = tid; i < own3; i += kNbThreads) {
+      const int m = i / own, j = i - m * own;
+      const double* w = A.w0 + 6 * (size_t)(first + (j < cnt ? j : 0));
+      S.q[i] = w[m];
+      S.p[i] = dir * w[3 + m];
+      S.ext[i] = 0.0;
+      S.Q[i] = S.q[i];
+    }
+    __syncthreads();
+    double tau = dir * A.t0;
+    const double tau1 = dir * A.t1;
+    int si = 0;
+    while (si < A.T && dir * A.ts[si] <= tau) save(si++, S.q, S.p);
+    int status = GX_SUCCESS;
+    long long nst = 0, nacc = 0;
+    const double nn = 6.0 * (double)n;
+    // Each trip publishes one set of positions, meets, and evaluates the
+    // field there: at the start, at the trial point of the first-step rule,
+    // at a stage, or at a step's end (with the step's error).
+    enum { kStart, kTrial, kStage, kEnd };
+    int phase = kStart, stage = 0;
+    double h = 0.0, hh = 0.0, d1 = 0.0, t_eval = dir * tau;
+    double tnext = tau, prev_inv = 1.0, prev_prev_inv = 1.0;
+    bool at_dtmin = false;
+    while (A.t0 != A.t1) {
+      double sq = 0.0, bad = 0.0;
+      const bool last = phase == kEnd && SF == M::S;  // Dopri5's end stage is done
+      settle();
+      for (int k = tid; k < own3; k += kNbThreads) {
+        const int m = k / own, j = k - m * own;
+        if (j >= cnt) continue;
+        double x = S.q[k];
+        if (phase == kTrial) {
+          x += S.p[k] * hh;
+        } else if (phase == kStage) {
+          // zero weights from `stage` on, where g holds the last step's
+          const double* a = S.aa + stage * M::S;
+          double s = 0.0;
+#pragma unroll
+          for (int l = 0; l < M::S - 1; ++l) s = fma(a[l], S.g[l * own3 + k], s);
+          x = fma(h, fma(K.rs[stage], S.p[k], h * s), x);
+        } else if (phase == kEnd) {
+          double b = 0.0, ba = 0.0, e = 0.0, ea = 0.0;
+#pragma unroll
+          for (int l = 0; l < M::S; ++l) {
+            const double gl = S.g[l * own3 + k];
+            b = fma(K.b[l], gl, b);
+            ba = fma(K.ba[l], gl, ba);
+            if (PID) {
+              e = fma(K.e[l], gl, e);
+              ea = fma(K.ea[l], gl, ea);
+            }
+          }
+          const double q0 = x, p0 = S.p[k];
+          x = fma(h, fma(K.sb, p0, h * ba), q0);
+          const double p1 = fma(h, b, p0);
+          S.q1[k] = x;
+          S.p1[k] = p1;
+          if (!isfinite(x) || !isfinite(p1)) bad = 1.0;
+          if (PID) {
+            const double eq = h * fma(K.se, p0, h * ea);
+            const double ep = h * e;
+            const double uq = eq / (A.atol + fmax(fabs(q0), fabs(x)) * A.rtol);
+            const double up = ep / (A.atol + fmax(fabs(p0), fabs(p1)) * A.rtol);
+            sq += uq * uq + up * up;
+          }
+        }
+        publish(m, j, x);
+      }
+      if (phase == kEnd) {
+        sum(sq, bad);
+        offer(sq, bad);
+      }
+      __syncthreads();
+      if (!last) external(t_eval);
+      bool keep = true;
+      double next_tau1 = 0.0;
+      if (phase == kEnd) {
+        total(sq, bad);
+        ++nst;
+        if (bad != 0.0) {
+          status = GX_NONFINITE;
+          break;
+        }
+        if (PID) {
+          const double scaled = sqrt(sq / nn);
+          keep = scaled < 1.0;
+          if (A.dtmin > 0.0) keep = keep || at_dtmin;
+          const double inv = 1.0 / scaled;
+          double f = (A.c1 == 0.0) ? 1.0 : pow(inv, A.c1);
+          if (A.c2 != 0.0) f *= pow(prev_inv, A.c2);
+          if (A.c3 != 0.0) f *= pow(prev_prev_inv, A.c3);
+          const double fmin_ = keep ? 1.0 : A.factormin;
+          const double factor = fmin(fmax(A.safety * f, fmin_), A.factormax);
+          double dt = fmin(h * factor, A.dtmax);
+          if (A.dtmin > 0.0) {
+            if (!A.force_dtmin && dt < A.dtmin) status = GX_DT_MIN_REACHED;
+            at_dtmin = dt <= A.dtmin;
+            dt = fmax(dt, A.dtmin);
+          }
+          if (keep) {
+            prev_prev_inv = prev_inv;
+            prev_inv = (inv == 0.0 || isinf(inv)) ? 1.0 : inv;
+          }
+          next_tau1 = (keep ? tnext : tau) + dt;
+        } else {
+          next_tau1 = tnext + A.dt0;
+        }
+      }
+      const bool field = keep && !last;
+      if (field) fetch();
+      close();
+      if (field) accelerate(S.g + (phase == kStart ? 0 : phase == kStage ? stage : SF - 1) * own3);
+      bool begin = false;  // the next trip begins a step
+      if (phase == kStart || phase == kTrial) {
+        // first step: dt0; dtmin if the controller sets one (as the orbit
+        // integrators); else diffrax's initial-step heuristic over the system
+        double h0 = A.dt0 > 0.0 ? A.dt0 : (PID && A.dtmin > 0.0 ? A.dtmin : 0.0);
+        if (!(h0 > 0.0)) {
+          double s0 = 0.0, s1 = 0.0;
+          for (int k = tid; k < own3; k += kNbThreads) {
+            if (k % own >= cnt) continue;
+            const double q = S.q[k], p = S.p[k], a = S.g[k];
+            const double wq = A.atol + fabs(q) * A.rtol, wp = A.atol + fabs(p) * A.rtol;
+            if (phase == kStart) {
+              s0 += (q / wq) * (q / wq) + (p / wp) * (p / wp);
+              s1 += (p / wq) * (p / wq) + (a / wp) * (a / wp);
+            } else {
+              const double u = ((p + dir * a * dir * hh) - p) / wq;
+              const double v = dir * (gend[k] - a) / wp;
+              s0 += u * u + v * v;
+            }
+          }
+          sum(s0, s1);
+          settle();
+          offer(s0, s1);
+          total(s0, s1);
+          close();
+          if (phase == kStart) {
+            const double d0 = sqrt(s0 / nn);
+            d1 = sqrt(s1 / nn);
+            const bool cond = (d0 < 1e-5) || (d1 < 1e-5);
+            hh = cond ? 1e-6 : 0.01 * (d0 / (cond ? 1.0 : d1));
+            phase = kTrial;
+            t_eval = dir * (tau + hh);
+            continue;
+          }
+          const double d2 = sqrt(s0 / nn) / hh;
+          const double maxd = fmax(d1, d2);
+          const double h1 = (maxd <= 1e-15) ? fmax(1e-6, hh * 1e-3)
+                                            : pow(0.01 / maxd, 1.0 / ((double)M::order + 1.0));
+          h0 = fmin(100.0 * hh, h1);
+        }
+        if (PID) {
+          h0 = fmin(h0, A.dtmax);
+          if (A.dtmin > 0.0) {
+            at_dtmin = h0 <= A.dtmin;
+            h0 = fmax(h0, A.dtmin);
+          }
+        }
+        tnext = fmin(tau + h0, tau1);
+        begin = true;
+      } else if (phase == kStage) {
+        if (++stage == M::S) {
+          phase = kEnd;
+          t_eval = dir * tnext;
+        } else {
+          t_eval = dir * fma(K.c[stage], h, tau);
+        }
+      } else {
+        if (keep) {
+          // saves in (tau, tnext]: the step end, or the step's dense output
+          while (si < A.T && dir * A.ts[si] <= tnext) {
+            const double ts_tau = dir * A.ts[si];
+            if (ts_tau == tnext)
+              save(si, S.q1, S.p1);
+            else
+              save_inside(si, (ts_tau - tau) / h, h);
+            ++si;
+          }
+          __syncthreads();
+          for (int k = tid; k < own3; k += kNbThreads) {
+            S.q[k] = S.q1[k];
+            S.p[k] = S.p1[k];
+            S.g[k] = gend[k];
+          }
+          ++nacc;
+        }
+        __syncthreads();
+        const double tprev = fmin(keep ? tnext : tau, tau1);
+        tnext =
+            (next_tau1 > tau1 - 1e-10) ? (keep ? tau1 : tprev + 0.5 * (tau1 - tprev)) : next_tau1;
+        tau = tprev;
+        if (status == GX_DT_MIN_REACHED) break;
+        begin = true;
+      }
+      if (begin) {
+        if (!(tau < tau1)) break;
+        if (nst >= A.max_steps) {
+          status = GX_MAX_STEPS_REACHED;
+          break;
+        }
+        h = tnext - tau;
+        if (!(h >= 0.0)) {
+          status = GX_NONFINITE;
+          break;
+        }
+        phase = kStage;
+        stage = 1;
+        t_eval = dir * fma(K.c[1], h, tau);
+      }
+    }
+    if (status != GX_SUCCESS) {
+      const double nanv = __longlong_as_double(0x7ff8000000000000ULL);
+      for (; si < A.T; ++si)
+        for (int j = tid; j < cnt; j += kNbThreads)
+          for (int m = 0; m < 6; ++m) A.out[((size_t)(first + j) * A.T + si) * 6 + m] = nanv;
+    }
+    if (blockIdx.x == 0 && tid == 0) {
+      if (A.status) *A.status = status;
+      if (A.nsteps) *A.nsteps = nst;
+      if (A.naccept) *A.naccept = nacc;
+    }
+  }
+};
+
+template <class M, bool PID, class E>
+__global__ void __launch_bounds__(kNbThreads) k_nbody_grid(DPot P, NArgs A, NGrid X) {
+  extern __shared__ double nb_lds[];
+  __shared__ double2 red[kNbWaves];
+  const int n = (int)A.n, own = X.own, o3 = 3 * X.own;
+  NbGridSolve<M, PID, E> R{P, A, X};
+  double* d = nb_lds;
+  R.S.x = d;
+  R.S.y = d + n;
+  R.S.z = d + 2 * n;
+  R.S.gm = d + 3 * n;
+  d += 4 * n;
+  R.S.q = d;
+  R.S.p = d + o3;
+  R.S.q1 = d + 2 * o3;
+  R.S.p1 = d + 3 * o3;
+  R.S.Q = d + 4 * o3;
+  R.S.ext = d + 5 * o3;
+  R.S.g = d + 6 * o3;
+  R.S.part = d + (6 + M::SF) * o3;
+  R.S.aa = R.S.part + 3 * (own > kNbWaves ? own : kNbWaves);
+  R.red = red;
+  R.n = n;
+  R.own = own;
+  R.tid = threadIdx.x;
+  R.first = blockIdx.x * own;
+  R.cnt = n - R.first < own ? n - R.first : own;
+  R.run();
+}
+
+// The system over workgroups: GX_OK when launched, 1 when the device cannot
+// hold them all at once (or the stream is being captured, which takes no
+// cooperative launch).
+template <class M, bool PID, class E>
+int launch_grid(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
+  const auto kern = k_nbody_grid<M, PID, E>;
+  NGrid X{};
+  X.own = A.n <= kNbOne ? (int)A.n : (int)((A.n + kNbGroups - 1) / kNbGroups);
+  if (A.n > kNbOne && X.own < kNbOwnMin) X.own = kNbOwnMin;
+  X.G = (int)((A.n + X.own - 1) / X.own);
+  // what G workgroups exchange (72 bytes a body, 48 a workgroup) fits where
+  // the one-workgroup kernel keeps its state (432 bytes a body)
+  X.pos = reinterpret_cast<NbSlot*>(static_cast<char*>(workspace) + 256);
+  X.part = X.pos + 9 * A.n;
+  const size_t lds = sizeof(double) * nb_lds_doubles(A.n, X.own, M::SF);
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return GX_ELAUNCH;
+  if (X.G == 1) {
+    hipLaunchKernelGGL(kern, dim3(1), dim3(kNbThreads), lds, s, ext->dev, A, X);
+    return check(hipGetLastError());
+  }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  int coop = 0, occ = 0;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ext->device) != hipSuccess ||
+      !coop ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, kNbThreads, lds) != hipSuccess ||
+      (long long)occ * num_cus(ext->device) < X.G) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  const long long slots = 9 * A.n + 6 * X.G;
+  hipLaunchKernelGGL(k_nb_empty, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, s, X.pos, slots);
+  DPot Pd = ext->dev;
+  NArgs Ad = A;
+  void* args[] = {&Pd, &Ad, &X};
+  if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kern), dim3(X.G), dim3(kNbThreads),
+                                 args, (unsigned)lds, s) == hipSuccess)
+    return GX_OK;
+  (void)hipGetLastError();
+  return 1;
+}
+
+template <class M, bool PID>
+int launch_nbody(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
+  const int rc = ext->sig == kSigMilkyWay ? launch_grid<M, PID, EvalMilkyWay>(ext, A, workspace, s)
+                                          : launch_grid<M, PID, EvalTable<true>>(ext, A, workspace, s);
+  if (rc != 1) return rc;
+  hipLaunchKernelGGL((k_nbody<M, PID>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
+  return check(hipGetLastError());
+}
+
 // The field alone (NBodyField.__call__'s acceleration): one thread per body,
 // positions staged through LDS in tiles.
 __global__ void __launch_bounds__(256) k_nbody_accel(DPot P, const double* __restrict__ xyz,
@@ -475,18 +1092,11 @@ int gx_nbody_integrate(const gx_pot* ext, const double* gm, double eps,
   A.G = w + 12 * n;
   hipStream_t s = (hipStream_t)stream;
   const bool pid = cfg->controller == GX_PID;
-  if (cfg->method == GX_DOPRI8) {
-    if (pid)
-      hipLaunchKernelGGL((k_nbody<Dopri8, true>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
-    else
-      hipLaunchKernelGGL((k_nbody<Dopri8, false>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
-  } else {
-    if (pid)
-      hipLaunchKernelGGL((k_nbody<Dopri5, true>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
-    else
-      hipLaunchKernelGGL((k_nbody<Dopri5, false>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
-  }
-  return check(hipGetLastError());
+  if (cfg->method == GX_DOPRI8)
+    return pid ? launch_nbody<Dopri8, true>(ext, A, workspace, s)
+               : launch_nbody<Dopri8, false>(ext, A, workspace, s);
+  return pid ? launch_nbody<Dopri5, true>(ext, A, workspace, s)
+             : launch_nbody<Dopri5, false>(ext, A, workspace, s);
 }
 
 }  // extern "C"

@@ -174,3 +174,79 @@ def test_gpu_nbody_backward_and_bad_sizes():
     big = gd.NBodyField(masses=np.ones(5000), eps=1e-3)
     with pytest.raises(_lib.GalaxHipError):
         gd.solve_nbody(big, (np.zeros((5000, 3)), np.zeros((5000, 3))), 0.0, 1.0, solver=solver, dt0=0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 48, 49, 51, 193, 1025, 1027])
+def test_gpu_nbody_split_over_workgroups(n):
+    """Sizes at the edges of the division among workgroups (one workgroup up
+    to 48 bodies; several of four or more, the last one ragged): fixed steps
+    with saves inside steps, at the bound of the fixed-step test above."""
+    w0, m = _cluster(n, 5, SMOOTH["mmax"] * 20.0 / max(n, 20))
+    mw = gp.MilkyWayPotential()
+    solver = gd.OrbitSolver(gd.Dopri8(), stepsize_controller=gd.ConstantStepSize(), max_steps=None)
+    ts = np.array([0.0, 0.33, 1.0, 2.2, 2.5])
+    print(f"[case] nbody split n={n}", flush=True)
+    field = gd.NBodyField(masses=m, eps=SMOOTH["eps"], external_potential=mw)
+    soln = gd.solve_nbody(field, (w0[:, :3], w0[:, 3:]), 0.0, 2.5, saveat=ts, solver=solver, dt0=0.5)
+    ref, st, ns, _ = oracle.nbody_integrate(mw, G * m, SMOOTH["eps"], solver, w0, 0.0, 2.5, ts=ts, dt0=0.5)
+    assert soln.status == 0 and st == 0 and soln.nsteps == ns == 5
+    got = np.concatenate([np.transpose(soln.ys[0], (1, 0, 2)), np.transpose(soln.ys[1], (1, 0, 2))], -1)
+    rel = np.abs(got - ref) / np.abs(ref).max(axis=(1, 2), keepdims=True)
+    assert rel.max() < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method", [gd.Dopri8(), gd.Dopri5()], ids=["dopri8", "dopri5"])
+def test_gpu_nbody_split_adaptive_steps_and_limits(method):
+    """The controller over several workgroups takes the oracle's steps, for a
+    table field too, and stops at max_steps as the oracle does."""
+    w0, m = _cluster(130, 6, SMOOTH["mmax"])
+    ext = gp.HernquistPotential(m_tot=1e12, r_s=10.0)
+    field = gd.NBodyField(masses=m, eps=SMOOTH["eps"], external_potential=ext)
+    solver = gd.OrbitSolver(method, stepsize_controller=gd.PIDController(rtol=1e-9, atol=1e-9), max_steps=None)
+    print("[case] nbody split adaptive", flush=True)
+    for t1, max_steps in ((20.0, "default"), (20.0, 3)):
+        kw = {} if max_steps == "default" else {"max_steps": max_steps}
+        soln = gd.solve_nbody(field, (w0[:, :3], w0[:, 3:]), 0.0, t1, saveat=[7.0, t1], solver=solver, **kw)
+        ref, st, ns, na = oracle.nbody_integrate(ext, G * m, SMOOTH["eps"], solver.with_(**kw) if kw else solver, w0,
+                                                 0.0, t1, ts=np.array([7.0, t1]))
+        assert (soln.status, soln.nsteps, soln.naccept) == (st, ns, na)
+        got = np.concatenate([np.transpose(soln.ys[0], (1, 0, 2)), np.transpose(soln.ys[1], (1, 0, 2))], -1)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+        assert np.nanmax(np.abs(got - ref), initial=0.0) < 1e-9 * np.nanmax(np.abs(ref), initial=1.0)
+
+
+@pytest.mark.gpu
+def test_gpu_nbody_under_capture_matches_the_direct_call():
+    """A captured solve (one workgroup: no cooperative launch in a graph),
+    replayed, against the direct one."""
+    import ctypes
+
+    import torch
+
+    from galax_amd import _lib
+
+    w0, m = _cluster(130, 7, SMOOTH["mmax"])
+    field = gd.NBodyField(masses=m, eps=SMOOTH["eps"], external_potential=gp.MilkyWayPotential())
+    solver = gd.OrbitSolver(gd.Dopri8(), stepsize_controller=gd.ConstantStepSize(), max_steps=None)
+    print("[case] nbody captured", flush=True)
+    direct = gd.solve_nbody(field, (w0[:, :3], w0[:, 3:]), 0.0, 2.0, solver=solver, dt0=0.5)
+    lib, cfg = _lib.lib(), solver.cfg(dt0=0.5)
+    w, gm = torch.as_tensor(w0, device="cuda"), field._gm(torch)
+    ts = torch.tensor([2.0], dtype=torch.float64, device="cuda")
+    out = torch.zeros(130, 1, 6, dtype=torch.float64, device="cuda")
+    ws = torch.zeros((int(lib.gx_nbody_workspace_bytes(130)) + 7) // 8, dtype=torch.float64, device="cuda")
+    ext = field.external_potential._handle()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rc = lib.gx_nbody_integrate(ext, _lib.ptr(gm), field.eps, ctypes.addressof(cfg), _lib.ptr(w), 0.0, 2.0,
+                                    _lib.ptr(ts), 1, 130, _lib.ptr(out), None, None, None, _lib.ptr(ws),
+                                    _lib.stream_ptr())
+        _lib.check(rc, "gx_nbody_integrate")
+    want = np.concatenate([direct.ys[0][0], direct.ys[1][0]], 1)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        got = out[:, 0].cpu().numpy()
+        assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()
