@@ -7,12 +7,12 @@
 // loss derivatives of tests/functional/test_mockstreamgenerator.py:24-116);
 // here the derivative of the discrete map is formed exactly, in reverse.
 //
-// Per orbit (one lane): a forward sweep stores the state every K steps; the
-// reverse sweep walks the checkpoint segments backwards, recomputes each
-// segment's states, and for every step recomputes its stage positions and
-// applies the adjoint of the step.  In Runge-Kutta-Nystrom form (stages Q_i,
-// accelerations g_i = a(Q_i), weights b, A, (bA), (A A)) the adjoint of one
-// step of size h with output cotangents (qb', pb') is
+// Per orbit (one lane of two waves): a forward sweep stores states, the
+// reverse sweep walks the steps backwards, and for every step recomputes its
+// stage positions and applies the adjoint of the step.  In Runge-Kutta-
+// Nystrom form (stages Q_i, accelerations g_i = a(Q_i), weights b, A, (bA),
+// (A A)) the adjoint of one step of size h with output cotangents (qb', pb')
+// is
 //   gb_j = h b_j pb' + h^2 (bA)_j qb'                 (all stages j)
 //   qb = qb',  pb = pb' + h (sum b) qb'
 //   for k = S-1 .. 0:
@@ -38,8 +38,19 @@
 namespace gx {
 namespace {
 
-constexpr int kAdjBlock = 128;
+// Orbits of a workgroup: two waves of them, and two more waves for the same
+// orbits (see k_adjoint).  One wave of each kind (64 orbits) was as fast
+// while every workgroup had a CU of its own, but two workgroups on a CU put
+// their second waves on the same SIMD (us a step at 20,000 orbits: 13.7
+// against 9.9).
+constexpr int kAdjOrbits = 128;
 constexpr int kMaxTheta = 12;  // 3 table parameters x up to 4 components
+
+// Up to here every step's start state is kept (56 bytes a step and orbit),
+// which saves a third of the forward work; beyond it every K-th, and a
+// segment of K steps is integrated again before it is reversed.  4 GiB, a
+// sixtieth of the device's memory, holds 25,000 orbits of 3,000 steps.
+constexpr long long kAllStatesBytes = 4LL << 30;
 
 struct AArgs {
   double dt0;
@@ -49,17 +60,17 @@ struct AArgs {
   int t_stride;
   int T;
   int ts_mode;
-  int K;            // checkpoint interval (steps)
-  long long C;      // checkpoint slots per orbit
+  int all;            // every step's state is kept: one segment
+  long long K;        // steps of a segment
+  long long limit;    // steps an orbit may take
   const double* ts;
   const double* cot;  // n x T x 6
   long long n;
   double* w0_bar;     // n x 6
   double* theta_bar;  // n x ntheta
   int ntheta;
-  double* ckpt;  // [C][7][n]
-  double* seg;   // [K][7][n]
-  double* stq;   // [SF][3][n]: stage positions and the end position q1
+  double* ckpt;  // [limit / K][7][n] segment starts (not `all`)
+  double* seg;   // [K][7][n] step starts of a segment
   int* status;
 };
 
@@ -82,11 +93,11 @@ __device__ __forceinline__ double clip_end(double tprev, double tnext,
   return (tnext > t1 - 1e-10) ? t1 : tnext;
 }
 
-// Forward step (no error estimate); optionally records the stage positions.
+// Forward step (no error estimate); optionally records the stage positions
+// and the step's end in this lane's column of st.
 template <class M, class E, bool REC>
-__device__ __forceinline__ void step_fwd(const DPot& P, const AArgs& A,
-                                         long long i, double h, double (&q)[3],
-                                         double (&p)[3]) {
+__device__ __forceinline__ void step_fwd(const DPot& P, double* st, double h,
+                                         double (&q)[3], double (&p)[3]) {
   constexpr int S = M::S;
   double g[S][3];
 #pragma unroll
@@ -114,7 +125,7 @@ __device__ __forceinline__ void step_fwd(const DPot& P, const AArgs& A,
     }
     if (REC) {
 #pragma unroll
-      for (int m = 0; m < 3; ++m) A.stq[((long long)k * 3 + m) * A.n + i] = Q[m];
+      for (int m = 0; m < 3; ++m) st[(k * 3 + m) * kAdjOrbits] = Q[m];
     }
     E::acc(P, Q[0], Q[1], Q[2], 0.0, g[k][0], g[k][1], g[k][2]);
   }
@@ -137,9 +148,9 @@ __device__ __forceinline__ void step_fwd(const DPot& P, const AArgs& A,
   const double q1 = fma(h, fma(sb, p[1], h * c1), q[1]);
   const double q2 = fma(h, fma(sb, p[2], h * c2), q[2]);
   if (REC && M::SF > S) {
-    A.stq[((long long)S * 3 + 0) * A.n + i] = q0;
-    A.stq[((long long)S * 3 + 1) * A.n + i] = q1;
-    A.stq[((long long)S * 3 + 2) * A.n + i] = q2;
+    st[(S * 3 + 0) * kAdjOrbits] = q0;
+    st[(S * 3 + 1) * kAdjOrbits] = q1;
+    st[(S * 3 + 2) * kAdjOrbits] = q2;
   }
   p[0] = fma(h, b0, p[0]);
   p[1] = fma(h, b1, p[1]);
@@ -149,62 +160,121 @@ __device__ __forceinline__ void step_fwd(const DPot& P, const AArgs& A,
   q[2] = q2;
 }
 
-// Sum over components of H w and (da/dtheta)^T w at Q.
-template <int... K, size_t... I>
-__device__ __forceinline__ void adj_all(const DPot& P, const double (&Q)[3],
-                                        const double (&w)[3], double (&Hw)[3],
-                                        double (&th)[kMaxTheta],
-                                        std::index_sequence<I...>) {
-  Hw[0] = Hw[1] = Hw[2] = 0.0;
-  (comp_adjoint<K>(P.comps[I], Q[0], Q[1], Q[2], w, Hw, th + 3 * I), ...);
+// What a lane carries from step to step: in the first set of waves (see
+// k_adjoint) a step's start state q, p and, in th[0], its time; in the second
+// the cotangents of a state and of the parameters.  One set of registers
+// serves both.
+struct Carry {
+  double q[3], p[3], th[kMaxTheta];
+};
+
+// State rows [7][n] in memory: q, p, tau of orbit i.
+__device__ __forceinline__ void put_state(double* row, long long n, long long i, const Carry& s) {
+  double* r = row + i;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    r[m * n] = s.q[m];
+    r[(m + 3) * n] = s.p[m];
+  }
+  r[6 * n] = s.th[0];
+}
+__device__ __forceinline__ void get_state(const double* row, long long n, long long i, Carry& s) {
+  const double* r = row + i;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    s.q[m] = r[m * n];
+    s.p[m] = r[(m + 3) * n];
+  }
+  s.th[0] = r[6 * n];
 }
 
-// Adjoint of one step of size h from (q, p) given the step end's output
-// cotangents (qb, pb), updated in place to the cotangents of (q, p).  The
-// save times inside the step add gx (their stage cotangents over the SF
-// slots) and dq, dp (their direct cotangents of q and p); with no such save
-// (any_save false) those are zero and the end stage is skipped.
-template <class M, class E, int... K>
-__device__ __forceinline__ void step_adj(const DPot& P, const AArgs& A,
-                                         long long i, double h,
-                                         const double (&q)[3],
-                                         const double (&p)[3], double (&qb)[3],
-                                         double (&pb)[3],
-                                         double (&th)[kMaxTheta],
-                                         const double (&gx)[M::SF][3],
-                                         const double (&dq)[3],
-                                         const double (&dp)[3],
-                                         bool any_save) {
+__device__ __forceinline__ int wave_max(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+__device__ __forceinline__ void add_save(const AArgs& A, long long i, int s, double dir, Carry& b) {
+  const double* c = A.cot + (i * A.T + s) * 6;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    b.q[m] += c[m];
+    b.p[m] += dir * c[m + 3];
+  }
+}
+
+// Adjoint of one step of size h, whose stage positions are in this lane's
+// column of st: b holds the cotangents of the step's end on entry and those
+// of its start on return.  Save times inside the step (their index counts
+// down in si) add to the stage and state cotangents; with none the end stage
+// is skipped.
+template <class M, class F>
+__device__ __forceinline__ void step_adj(const DPot& P, const AArgs& A, const double* st,
+                                         long long i, double dir, double t0v, double t1v,
+                                         double tau, double tau1, int& si, Carry& b) {
   constexpr int S = M::S;
   constexpr int SF = M::SF;
-  {
-    double qq[3] = {q[0], q[1], q[2]}, pp[3] = {p[0], p[1], p[2]};
-    step_fwd<M, E, true>(P, A, i, h, qq, pp);
-  }
+  const double h = tau1 - tau, h2 = h * h;
   double gb[SF][3];
-  const double h2 = h * h;
 #pragma unroll
   for (int j = 0; j < SF; ++j)
 #pragma unroll
     for (int m = 0; m < 3; ++m)
-      gb[j][m] = (j < S ? fma(h * M::k.b[j], pb[m], h2 * M::k.ba[j] * qb[m]) : 0.0) + gx[j][m];
+      gb[j][m] = j < S ? fma(h * M::k.b[j < S ? j : 0], b.p[m], h2 * M::k.ba[j < S ? j : 0] * b.q[m])
+                       : 0.0;
   constexpr double sb = M::k.sb;
 #pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    pb[m] = fma(h * sb, qb[m], pb[m]) + dp[m];
-    qb[m] += dq[m];
+  for (int m = 0; m < 3; ++m) b.p[m] = fma(h * sb, b.q[m], b.p[m]);
+  // saves inside: the step's dense output at th = (t_s - tau) / h
+  bool any_save = false;
+  while (si >= 0) {
+    const double tsv = dir * save_time_a(A, i, si, t0v, t1v);
+    if (!(tsv > tau && tsv < tau1)) break;
+    const double* c = A.cot + (i * A.T + si) * 6;
+    const double cq[3] = {c[0], c[1], c[2]}, cp[3] = {dir * c[3], dir * c[4], dir * c[5]};
+    const double tht = (tsv - tau) / h;
+    const double ht = h * tht, hht = h * ht;
+    // one stage's weights at a time: all of them at once do not fit beside
+    // the stage cotangents
+    constexpr int D = sizeof(M::dn.wq[0]) / sizeof(double);
+    ConstDouble* tq = table_here(&M::dn.wq[0][0]);
+    ConstDouble* tp = table_here(&M::dn.wp[0][0]);
+#pragma unroll
+    for (int l = 0; l < SF; ++l) {
+      if (M::dn.nq[l]) {
+        const double w = hht * horner_here<D>(tq + D * l, tht);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) gb[l][m] = fma(w, cq[m], gb[l][m]);
+      }
+      if (M::dn.np[l]) {
+        const double w = ht * horner_here<D>(tp + D * l, tht);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) gb[l][m] = fma(w, cp[m], gb[l][m]);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      b.q[m] += cq[m];
+      b.p[m] = fma(ht, cq[m], b.p[m] + cp[m]);
+    }
+    any_save = true;
+    --si;
   }
+  auto stage = [&](int k, const double (&w)[3], double (&Hw)[3]) {
+    double Q[3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) Q[m] = st[(k * 3 + m) * kAdjOrbits];
+    F::adjoint(P, Q, w, Hw, b.th);
+  };
   if constexpr (SF > S) {
     if (any_save) {
       // the end stage g_E = a(q1), q1 = q + h (sb p + h sum (bA)_j g_j)
-      double Q[3], Hw[3];
-#pragma unroll
-      for (int m = 0; m < 3; ++m) Q[m] = A.stq[((long long)S * 3 + m) * A.n + i];
-      adj_all<K...>(P, Q, gb[S], Hw, th, std::make_index_sequence<sizeof...(K)>{});
+      double Hw[3];
+      stage(S, gb[S], Hw);
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
-        qb[m] -= Hw[m];
-        pb[m] = fma(-h * sb, Hw[m], pb[m]);
+        b.q[m] -= Hw[m];
+        b.p[m] = fma(-h * sb, Hw[m], b.p[m]);
       }
 #pragma unroll
       for (int j = 0; j < S; ++j) {
@@ -218,209 +288,197 @@ __device__ __forceinline__ void step_adj(const DPot& P, const AArgs& A,
   }
 #pragma unroll
   for (int k = S - 1; k >= 0; --k) {
-    double Q[3], Hw[3];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) Q[m] = A.stq[((long long)k * 3 + m) * A.n + i];
-    adj_all<K...>(P, Q, gb[k], Hw, th, std::make_index_sequence<sizeof...(K)>{});
+    double Hw[3];
+    stage(k, gb[k], Hw);
     // Qb_k = -H gb_k
     const double rs = M::k.rs[k];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-      qb[m] -= Hw[m];
-      pb[m] = fma(-h * rs, Hw[m], pb[m]);
+      b.q[m] -= Hw[m];
+      b.p[m] = fma(-h * rs, Hw[m], b.p[m]);
+      Hw[m] *= -h2;
     }
 #pragma unroll
     for (int j = 0; j < k; ++j) {
       const double a = M::k.aa[k][j];
       if (a != 0.0) {
 #pragma unroll
-        for (int m = 0; m < 3; ++m) gb[j][m] = fma(-h2 * a, Hw[m], gb[j][m]);
+        for (int m = 0; m < 3; ++m) gb[j][m] = fma(a, Hw[m], gb[j][m]);
       }
     }
   }
 }
 
-template <class M, class E, int... K>
-__global__ void __launch_bounds__(kAdjBlock) k_adjoint(DPot P, AArgs A) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A.n) return;
-  const double t0v = A.t0[A.t_stride ? i : 0];
-  const double t1v = A.t1[A.t_stride ? i : 0];
+// Two sets of waves share a workgroup's orbits.  A step back needs its stage positions (13
+// field evaluations from the step's start state, independent of the
+// cotangents) and then 13 Hessian-vector products with the parameter
+// partials, one after the other.  The first set recomputes the positions
+// of one step into LDS while the second reverses the step after it, from the
+// other of two buffers.  A stream fit's orbits fill a third of the device's
+// SIMDs, so the second set costs nothing there.  Bound by instructions in
+// flight of one wave per SIMD: a step takes 4.4 us forward and 5.5 us back
+// up to 32,768 orbits (32.5 us in all with one set, IEEE divisions, 400
+// spilled registers and the stage positions in HBM); 131,072 orbits, which
+// fill the device, take 39 us a step (70).  20,000 orbits of up to 1,000
+// steps: 39.0 ms before, 12.2 ms.
+// The kernels' registers are checked in the tests: with spills the compiler
+// has stored a spilled parameter cotangent before restoring the execution
+// mask after a divergent loop, so that it was lost in some lanes.
+template <class M, class F>
+__global__ void __launch_bounds__(2 * kAdjOrbits)
+    __attribute__((amdgpu_waves_per_eu(2))) k_adjoint(DPot P, AArgs A) {
+  __shared__ double st[2][3 * M::SF + 1][kAdjOrbits];  // stage positions, tau
+  __shared__ int steps[kAdjOrbits], stat[kAdjOrbits];
+  const int lane = threadIdx.x & (kAdjOrbits - 1);  // the orbit in the workgroup
+  const bool first = __builtin_amdgcn_readfirstlane(threadIdx.x) < kAdjOrbits;
+  const long long i = (long long)blockIdx.x * kAdjOrbits + lane;
+  const bool valid = i < A.n;
+  const long long ic = valid ? i : 0;
+  const double t0v = A.t0[A.t_stride ? ic : 0];
+  const double t1v = A.t1[A.t_stride ? ic : 0];
   const double dir = (t0v < t1v) ? 1.0 : -1.0;
-  const double tau0 = dir * t0v, tau1 = dir * t1v;
-  const double* w = A.w0 + i * 6;
-  double q[3] = {w[0], w[1], w[2]};
-  double p[3] = {dir * w[3], dir * w[4], dir * w[5]};
-  double th[kMaxTheta];
-#pragma unroll
-  for (int k = 0; k < kMaxTheta; ++k) th[k] = 0.0;
+  const double tau1 = dir * t1v;
+  // the end of step n from its start
+  auto next_tau = [&](long long n, double tau) {
+    return n == 0 ? fmin(tau + A.dt0, tau1) : clip_end(tau, tau + A.dt0, tau1);
+  };
 
-  // ---- forward sweep with checkpoints every K steps
-  long long N = 0;
-  double tau = tau0;
-  int status = GX_SUCCESS;
-  if (t0v != t1v) {
-    double tn = fmin(tau + A.dt0, tau1);
-    while (tau < tau1) {
-      if (N % A.K == 0) {
-        const long long c = N / A.K;
-        if (c >= A.C) {
-          status = GX_MAX_STEPS_REACHED;
-          break;
-        }
-        double* ck = A.ckpt + c * 7 * A.n + i;
-        ck[0 * A.n] = q[0];
-        ck[1 * A.n] = q[1];
-        ck[2 * A.n] = q[2];
-        ck[3 * A.n] = p[0];
-        ck[4 * A.n] = p[1];
-        ck[5 * A.n] = p[2];
-        ck[6 * A.n] = tau;
+  Carry s;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) s.q[m] = s.p[m] = 0.0;
+#pragma unroll
+  for (int k = 0; k < kMaxTheta; ++k) s.th[k] = 0.0;
+  // ---- forward sweep, by the first set
+  if (first) {
+    long long N = 0;
+    int status = GX_SUCCESS;
+    const double* w = A.w0 + ic * 6;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      s.q[m] = w[m];
+      s.p[m] = dir * w[3 + m];
+    }
+    double tau = dir * t0v;
+    long long in_seg = 0;
+    while (valid && t0v != t1v && tau < tau1) {
+      if (N >= A.limit) {
+        status = GX_MAX_STEPS_REACHED;
+        break;
       }
-      step_fwd<M, E, false>(P, A, i, tn - tau, q, p);
+      s.th[0] = tau;
+      if (A.all)
+        put_state(A.seg + N * 7 * A.n, A.n, i, s);
+      else if (in_seg == 0)
+        put_state(A.ckpt + N / A.K * 7 * A.n, A.n, i, s);
+      in_seg = in_seg + 1 == A.K ? 0 : in_seg + 1;
+      const double tn = next_tau(N, tau);
+      step_fwd<M, F, false>(P, nullptr, tn - tau, s.q, s.p);
       ++N;
       tau = tn;
-      tn = clip_end(tau, tau + A.dt0, tau1);
     }
+    steps[lane] = status == GX_SUCCESS ? (int)N : 0;
+    stat[lane] = status;
   }
+  __syncthreads();
+  const long long N = steps[lane];
+  const int status = stat[lane];
+
   // ---- reverse sweep
-  double qb[3] = {0.0, 0.0, 0.0}, pb[3] = {0.0, 0.0, 0.0};
   int si = A.T - 1;
-  auto cot = [&](int s, double (&cq)[3], double (&cp)[3]) {
-    const double* c = A.cot + (i * A.T + s) * 6;
-    cq[0] = c[0];
-    cq[1] = c[1];
-    cq[2] = c[2];
-    cp[0] = dir * c[3];
-    cp[1] = dir * c[4];
-    cp[2] = dir * c[5];
-  };
-  if (status == GX_SUCCESS) {
-    const long long nseg = (N + A.K - 1) / A.K;
-    for (long long c = nseg - 1; c >= 0; --c) {
-      // recompute the segment's step starts
-      const long long n0 = c * A.K;
-      const int len = (int)((N - n0) < A.K ? (N - n0) : A.K);
-      double qs[3], ps[3];
-      const double* ck = A.ckpt + c * 7 * A.n + i;
-      for (int m = 0; m < 3; ++m) {
-        qs[m] = ck[m * A.n];
-        ps[m] = ck[(m + 3) * A.n];
-      }
-      double ts_ = ck[6 * A.n];
+  const long long nseg = (N + A.K - 1) / A.K;
+  // trip counts that every wave agrees on: the longest orbit's
+  const int other = steps[lane ^ 64];
+  const int trips = wave_max((int)((max((int)N, other) + A.K - 1) / A.K));
+  for (int it = 0; it < trips; ++it) {
+    const long long c = nseg - 1 - it;
+    const long long n0 = c * A.K;
+    const int len = c < 0 ? 0 : (int)(N - n0 < A.K ? N - n0 : A.K);
+    const long long oc = (other + A.K - 1) / A.K - 1 - it;
+    const int olen = oc < 0 ? 0 : (int)(other - oc * A.K < A.K ? other - oc * A.K : A.K);
+    const int longest = wave_max(max(len, olen));
+    if (first && !A.all && len > 0) {
+      // the segment's step starts again
+      get_state(A.ckpt + c * 7 * A.n, A.n, i, s);
       for (int m = 0; m < len; ++m) {
-        double* sg = A.seg + (long long)m * 7 * A.n + i;
-        sg[0 * A.n] = qs[0];
-        sg[1 * A.n] = qs[1];
-        sg[2 * A.n] = qs[2];
-        sg[3 * A.n] = ps[0];
-        sg[4 * A.n] = ps[1];
-        sg[5 * A.n] = ps[2];
-        sg[6 * A.n] = ts_;
+        put_state(A.seg + (long long)m * 7 * A.n, A.n, i, s);
         if (m + 1 < len) {
-          const double tn = (n0 + m == 0) ? fmin(ts_ + A.dt0, tau1)
-                                          : clip_end(ts_, ts_ + A.dt0, tau1);
-          step_fwd<M, E, false>(P, A, i, tn - ts_, qs, ps);
-          ts_ = tn;
+          const double tn = next_tau(n0 + m, s.th[0]);
+          step_fwd<M, F, false>(P, nullptr, tn - s.th[0], s.q, s.p);
+          s.th[0] = tn;
         }
-      }
-      // reverse over the segment's steps
-      for (int m = len - 1; m >= 0; --m) {
-        const double* sg = A.seg + (long long)m * 7 * A.n + i;
-        const double qn[3] = {sg[0], sg[A.n], sg[2 * A.n]};
-        const double pn[3] = {sg[3 * A.n], sg[4 * A.n], sg[5 * A.n]};
-        const double tau_n = sg[6 * A.n];
-        const long long n = n0 + m;
-        const double tau_np1 = (n == 0) ? fmin(tau_n + A.dt0, tau1)
-                                        : clip_end(tau_n, tau_n + A.dt0, tau1);
-        // saves at the step end
-        while (si >= 0 && dir * save_time_a(A, i, si, t0v, t1v) == tau_np1) {
-          double cq[3], cp[3];
-          cot(si, cq, cp);
-          for (int k = 0; k < 3; ++k) {
-            qb[k] += cq[k];
-            pb[k] += cp[k];
-          }
-          --si;
-        }
-        // interior saves: the step's dense output at th = (t_s - tau_n) / h
-        const double h = tau_np1 - tau_n;
-        double gx[M::SF][3], dq[3] = {0.0, 0.0, 0.0}, dp[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-        for (int l = 0; l < M::SF; ++l) gx[l][0] = gx[l][1] = gx[l][2] = 0.0;
-        bool any_save = false;
-        while (si >= 0) {
-          const double tsv = dir * save_time_a(A, i, si, t0v, t1v);
-          if (!(tsv > tau_n && tsv < tau_np1)) break;
-          double cq[3], cp[3];
-          cot(si, cq, cp);
-          const double tht = (tsv - tau_n) / h;
-          double wq[M::SF], wp[M::SF];
-          dense_weights<M>(tht, wq, wp);
-          const double ht = h * tht, hht = h * ht;
-#pragma unroll
-          for (int l = 0; l < M::SF; ++l)
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-              gx[l][k] = fma(hht * wq[l], cq[k], fma(ht * wp[l], cp[k], gx[l][k]));
-          for (int k = 0; k < 3; ++k) {
-            dq[k] += cq[k];
-            dp[k] = fma(ht, cq[k], dp[k] + cp[k]);
-          }
-          any_save = true;
-          --si;
-        }
-        step_adj<M, E, K...>(P, A, i, h, qn, pn, qb, pb, th, gx, dq, dp, any_save);
       }
     }
-    // saves at (or before) the start
-    while (si >= 0) {
-      double cq[3], cp[3];
-      cot(si, cq, cp);
-      for (int k = 0; k < 3; ++k) {
-        qb[k] += cq[k];
-        pb[k] += cp[k];
+    if (first && len > 0) get_state(A.seg + (long long)(len - 1) * 7 * A.n, A.n, i, s);
+    for (int k = 0; k <= longest; ++k) {
+      if (first) {
+        const int m = len - 1 - k;
+        if (m >= 0) {
+          Carry ahead = s;
+          if (m > 0) get_state(A.seg + (long long)(m - 1) * 7 * A.n, A.n, i, ahead);
+          double* col = &st[k & 1][0][lane];
+          col[3 * M::SF * kAdjOrbits] = s.th[0];
+          step_fwd<M, F, true>(P, col, next_tau(n0 + m, s.th[0]) - s.th[0], s.q, s.p);
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            s.q[j] = ahead.q[j];
+            s.p[j] = ahead.p[j];
+          }
+          s.th[0] = ahead.th[0];
+        }
+      } else {
+        const int m = len - k;
+        if (k > 0 && m >= 0) {
+          const double* col = &st[(k - 1) & 1][0][lane];
+          const double tau = col[3 * M::SF * kAdjOrbits];
+          const double tau_e = next_tau(n0 + m, tau);
+          // saves at the step end
+          while (si >= 0 && dir * save_time_a(A, i, si, t0v, t1v) == tau_e) add_save(A, i, si--, dir, s);
+          step_adj<M, F>(P, A, col, i, dir, t0v, t1v, tau, tau_e, si, s);
+        }
       }
-      --si;
+      __syncthreads();
     }
   }
+  if (first || !valid) return;
+  // saves at (or before) the start
+  if (status == GX_SUCCESS)
+    while (si >= 0) add_save(A, i, si--, dir, s);
   double* wb = A.w0_bar + i * 6;
-  wb[0] = qb[0];
-  wb[1] = qb[1];
-  wb[2] = qb[2];
-  wb[3] = dir * pb[0];
-  wb[4] = dir * pb[1];
-  wb[5] = dir * pb[2];
-  for (int k = 0; k < A.ntheta && k < kMaxTheta; ++k)
-    A.theta_bar[i * A.ntheta + k] = th[k];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    wb[m] = s.q[m];
+    wb[3 + m] = dir * s.p[m];
+  }
+#pragma unroll
+  for (int k = 0; k < kMaxTheta; ++k)
+    if (k < A.ntheta) A.theta_bar[i * A.ntheta + k] = s.th[k];
   if (A.status) A.status[i] = status;
 }
 
-template <class M, int... K>
+template <class M, class F>
 int launch_adj(const gx_pot* pot, AArgs& A, hipStream_t s) {
-  using E = EvalFixed<K...>;
-  const long long blocks = (A.n + kAdjBlock - 1) / kAdjBlock;
-  hipLaunchKernelGGL((k_adjoint<M, E, K...>), dim3((unsigned)blocks),
-                     dim3(kAdjBlock), 0, s, pot->dev, A);
+  const long long blocks = (A.n + kAdjOrbits - 1) / kAdjOrbits;
+  if (blocks > 0x7fffffffLL) return GX_EINVAL;
+  hipLaunchKernelGGL((k_adjoint<M, F>), dim3((unsigned)blocks), dim3(2 * kAdjOrbits), 0, s,
+                     pot->dev, A);
   return check(hipGetLastError());
 }
 
 template <class M>
 int dispatch_adj(const gx_pot* pot, AArgs& A, hipStream_t s) {
-  if (pot->sig == kSigMilkyWay)
-    return launch_adj<M, GX_MIYAMOTO_NAGAI, GX_NFW, GX_HERNQUIST, GX_HERNQUIST>(pot, A, s);
+  if (pot->sig == kSigMilkyWay) return launch_adj<M, AdjointMW>(pot, A, s);
   if (pot->ncomp == 1 && pot->basic) {
     switch (pot->kind0) {
       case GX_KEPLER:
-        return launch_adj<M, GX_KEPLER>(pot, A, s);
+        return launch_adj<M, AdjointFixed<GX_KEPLER>>(pot, A, s);
       case GX_HERNQUIST:
-        return launch_adj<M, GX_HERNQUIST>(pot, A, s);
+        return launch_adj<M, AdjointFixed<GX_HERNQUIST>>(pot, A, s);
       case GX_MIYAMOTO_NAGAI:
-        return launch_adj<M, GX_MIYAMOTO_NAGAI>(pot, A, s);
+        return launch_adj<M, AdjointFixed<GX_MIYAMOTO_NAGAI>>(pot, A, s);
       case GX_NFW:
-        return launch_adj<M, GX_NFW>(pot, A, s);
+        return launch_adj<M, AdjointFixed<GX_NFW>>(pot, A, s);
       case GX_PLUMMER:
-        return launch_adj<M, GX_PLUMMER>(pot, A, s);
+        return launch_adj<M, AdjointFixed<GX_PLUMMER>>(pot, A, s);
       default:
         break;
     }
@@ -433,12 +491,23 @@ int dispatch_adj(const gx_pot* pot, AArgs& A, hipStream_t s) {
 
 using namespace gx;
 
+namespace {
+
+// Steps an orbit may take: whole segments, at least max_steps.
+int64_t step_limit(int64_t max_steps, int64_t K) { return (max_steps / K + 2) * K; }
+
+bool all_states(int64_t n, int64_t max_steps, int64_t K) {
+  return n == 0 || step_limit(max_steps, K) <= kAllStatesBytes / 56 / n;
+}
+
+}  // namespace
+
 extern "C" {
 
 int64_t gx_adjoint_workspace_bytes(int64_t n, int64_t max_steps, int32_t K) {
   if (n < 0 || max_steps < 0 || K < 1) return 0;
-  const int64_t C = max_steps / K + 2;
-  return 8 * n * (7 * C + 7 * (int64_t)K + 3 * 14) + 256;
+  return all_states(n, max_steps, K) ? 56 * n * step_limit(max_steps, K) + 256
+                                     : 56 * n * (max_steps / K + 2 + K) + 256;
 }
 
 int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
@@ -465,8 +534,9 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
   A.t_stride = t_stride;
   A.T = T;
   A.ts_mode = ts_mode;
-  A.K = K;
-  A.C = max_steps / K + 2;
+  A.limit = step_limit(max_steps, K);
+  A.all = all_states(n, max_steps, K) ? 1 : 0;
+  A.K = A.all ? A.limit : K;
   A.ts = ts;
   A.cot = cot;
   A.n = n;
@@ -476,8 +546,7 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
   A.status = status;
   char* ws = static_cast<char*>(workspace);
   A.ckpt = reinterpret_cast<double*>(ws);
-  A.seg = A.ckpt + 7 * A.C * n;
-  A.stq = A.seg + 7 * (long long)K * n;
+  A.seg = A.all ? A.ckpt : A.ckpt + 7 * (A.limit / K) * n;
   hipStream_t s = (hipStream_t)stream;
   if (cfg->method == GX_DOPRI8) return dispatch_adj<Dopri8>(pot, A, s);
   return dispatch_adj<Dopri5>(pot, A, s);

@@ -1133,6 +1133,36 @@ struct EvalMilkyWayPieces : EvalMilkyWayTracked {
 // and add (da/dtheta_k) . w to th[k] for the component's table parameters
 // theta = (p0, p1, p2) as given in gx_component (G m, then the lengths).
 // The raw table parameters sit in DComp::p[5..7] (see derive()).
+
+// The Miyamoto-Nagai disk's share, in terms of v = (x, y, A z / S) with
+// S = sqrt(z^2 + b^2), A = a + S, D = x^2 + y^2 + A^2 (grad Phi =
+// G M v / D^(3/2)):
+//   H w = G M [w' / D^(3/2) - 3 (v . w) v / D^(5/2)],
+//   w' = (w_x, w_y, (z^2 / S^2 + A b^2 / S^3) w_z),
+//   (da/da_param) . w = G M [3 A (v . w) / D^(5/2) - (z / S) w_z / D^(3/2)],
+//   (da/db) . w = (b / S) G M [3 A (v . w) / D^(5/2)
+//                              - (z / S) (1 - A / S) w_z / D^(3/2)].
+__device__ __forceinline__ void mn_adjoint(double GM, double a, double b,
+                                           double x, double y, double z,
+                                           const double (&w)[3],
+                                           double (&Hw)[3], double* th) {
+  const double S2 = z * z + b * b;
+  const double iS = rsqrt_fast(S2);
+  const double A = a + S2 * iS;
+  const double iD = rsqrt_fast(x * x + y * y + A * A);
+  const double iD2 = iD * iD, iD3 = iD2 * iD;
+  const double zS = z * iS, bS = b * iS, Az = A * zS;
+  const double vw = x * w[0] + y * w[1] + Az * w[2];
+  const double t3 = GM * iD3, t5 = 3.0 * t3 * iD2 * vw;
+  Hw[0] += t3 * w[0] - t5 * x;
+  Hw[1] += t3 * w[1] - t5 * y;
+  Hw[2] += t3 * (zS * zS + A * iS * bS * bS) * w[2] - t5 * Az;
+  const double t5A = t5 * A, tz = t3 * zS * w[2];
+  th[0] -= vw * iD3;
+  th[1] += t5A - tz;
+  th[2] += bS * (t5A - tz * (1.0 - A * iS));
+}
+
 template <int K>
 __device__ __forceinline__ void comp_adjoint(const DComp& c, double x,
                                              double y, double z,
@@ -1140,60 +1170,34 @@ __device__ __forceinline__ void comp_adjoint(const DComp& c, double x,
                                              double (&Hw)[3], double* th) {
   const double GM = c.p[5];
   if constexpr (K == GX_MIYAMOTO_NAGAI) {
-    const double a = c.p[6], b = c.p[7];
-    const double S2 = z * z + b * b, S = sqrt(S2);
-    const double A = a + S;
-    const double D2 = x * x + y * y + A * A, D = sqrt(D2);
-    const double iD3 = 1.0 / (D2 * D), iD5 = iD3 / D2;
-    const double iS = 1.0 / S;
-    const double Az = A * z * iS;
-    const double hxx = GM * (iD3 - 3.0 * x * x * iD5);
-    const double hyy = GM * (iD3 - 3.0 * y * y * iD5);
-    const double hxy = -3.0 * GM * x * y * iD5;
-    const double hxz = -3.0 * GM * x * Az * iD5;
-    const double hyz = -3.0 * GM * y * Az * iD5;
-    const double hzz = GM * (z * z * iD3 * iS * iS + A * b * b * iD3 * iS * iS * iS -
-                             3.0 * Az * Az * iD5);
-    Hw[0] += hxx * w[0] + hxy * w[1] + hxz * w[2];
-    Hw[1] += hxy * w[0] + hyy * w[1] + hyz * w[2];
-    Hw[2] += hxz * w[0] + hyz * w[1] + hzz * w[2];
-    // da/dGM = a/GM
-    th[0] -= (x * w[0] + y * w[1] + Az * w[2]) * iD3;
-    // da/da_param
-    th[1] -= GM * (-3.0 * A * iD5 * (x * w[0] + y * w[1]) +
-                   (z * iS * iD3 - 3.0 * z * A * A * iS * iD5) * w[2]);
-    // da/db
-    th[2] -= GM * (-3.0 * A * b * iS * iD5 * (x * w[0] + y * w[1]) +
-                   z * (b * iS * iS * iD3 - A * b * iS * iS * iS * iD3 -
-                        3.0 * A * A * b * iS * iS * iD5) *
-                       w[2]);
+    mn_adjoint(GM, c.p[6], c.p[7], x, y, z, w, Hw, th);
   } else {
     const double r2 = x * x + y * y + z * z + kTiny;
-    const double r = sqrt(r2), ir = 1.0 / r;
-    double d1, d2, drs;  // Phi', Phi'', d(Phi'/r)/d r_s
+    const double ir = rsqrt_fast(r2), r = r2 * ir;
+    double g, k, drs;  // Phi'/r, (Phi'' - Phi'/r) / r^2, d(Phi'/r)/d r_s
     if constexpr (K == GX_KEPLER) {
-      d1 = GM * ir * ir;
-      d2 = -2.0 * GM * ir * ir * ir;
+      g = GM * ir * ir * ir;
+      k = -3.0 * g * ir * ir;
       drs = 0.0;
     } else if constexpr (K == GX_HERNQUIST) {
-      const double rs = c.p[6], u = 1.0 / (r + rs);
-      d1 = GM * u * u;
-      d2 = -2.0 * GM * u * u * u;
-      drs = -2.0 * GM * u * u * u * ir;
+      const double u = rcp(r + c.p[6]);
+      g = GM * u * u * ir;
+      k = -g * ir * (2.0 * u + ir);
+      drs = -2.0 * g * u;
     } else if constexpr (K == GX_NFW) {
-      const double rs = c.p[6], u = 1.0 / (r + rs), L = log1p(r / rs);
-      d1 = GM * (L * ir * ir - u * ir);
-      d2 = GM * (u * ir * ir - 2.0 * L * ir * ir * ir + (2.0 * r + rs) * u * u * ir * ir);
-      drs = -GM * u * u * ir / rs;
+      const double rs = c.p[6], u = rcp(r + rs);
+      const double t = log1p_fast(r * c.p[2]) * ir - u;
+      g = GM * ir * ir * t;
+      k = GM * ir * ir * ir * ir * (r * u * u - 3.0 * t);
+      drs = -GM * u * u * ir * c.p[2];
     } else {  // Plummer
-      const double rs = c.p[6], d = r2 + rs * rs, id = 1.0 / sqrt(d);
-      d1 = GM * r * id * id * id;
-      d2 = GM * (rs * rs - 2.0 * r2) * id * id * id * id * id;
-      drs = -3.0 * GM * rs * id * id * id * id * id;
+      const double rs = c.p[6], id = rsqrt_fast(r2 + rs * rs);
+      g = GM * id * id * id;
+      k = -3.0 * g * id * id;
+      drs = rs * k;
     }
-    const double g = d1 * ir;  // a = -g x
+    // a = -g x
     const double xw = x * w[0] + y * w[1] + z * w[2];
-    const double k = (d2 - g) * ir * ir;
     Hw[0] += g * w[0] + k * xw * x;
     Hw[1] += g * w[1] + k * xw * y;
     Hw[2] += g * w[2] + k * xw * z;
@@ -1201,6 +1205,71 @@ __device__ __forceinline__ void comp_adjoint(const DComp& c, double x,
     if constexpr (K != GX_KEPLER) th[1] -= drs * xw;
   }
 }
+
+// The adjoint's field for a fixed sequence of origin-centred models: the
+// acceleration for the forward steps, and at Q for a cotangent w of it H w
+// and (da/dtheta) . w (three parameters a component).
+template <int... K>
+struct AdjointFixed : EvalFixed<K...> {
+  template <size_t... I>
+  __device__ __forceinline__ static void all(const DPot& P,
+                                             const double (&Q)[3],
+                                             const double (&w)[3],
+                                             double (&Hw)[3], double* th,
+                                             std::index_sequence<I...>) {
+    (comp_adjoint<K>(P.comps[I], Q[0], Q[1], Q[2], w, Hw, th + 3 * I), ...);
+  }
+  __device__ __forceinline__ static void adjoint(const DPot& P,
+                                                 const double (&Q)[3],
+                                                 const double (&w)[3],
+                                                 double (&Hw)[3], double* th) {
+    Hw[0] = Hw[1] = Hw[2] = 0.0;
+    all(P, Q, w, Hw, th, std::make_index_sequence<sizeof...(K)>{});
+  }
+};
+
+// The Milky Way model's, with what EvalMW shares between its spherical
+// components (one rsqrt, one reciprocal, one log1p): their Hessians are
+// g I + k x x^T, so the sums of g and k over the three serve H w.
+struct AdjointMW : EvalMW {
+  __device__ __forceinline__ static void adjoint(const DPot& P,
+                                                 const double (&Q)[3],
+                                                 const double (&w)[3],
+                                                 double (&Hw)[3], double* th) {
+    const double* dk = P.comps[0].p;
+    const double* hk = P.comps[1].p;
+    const double* bk = P.comps[2].p;
+    const double* nk = P.comps[3].p;
+    const double x = Q[0], y = Q[1], z = Q[2];
+    const double r2 = x * x + y * y + z * z + kTiny;
+    const double ir = rsqrt_fast(r2), r = r2 * ir, ir2 = ir * ir;
+    const double dh = r + hk[1], db = r + bk[1], dn = r + nk[1];
+    const double dbn = db * dn;
+    const double R = rcp(dh * dbn);
+    const double dR = dh * R;
+    const double uh = dbn * R, ub = dn * dR, un = db * dR;
+    const double uh2 = uh * uh;
+    const double t = log1p_inv(r * hk[2], hk[1] * uh) * ir - uh;
+    const double gh = ir2 * t;             // Phi'/r over G m
+    const double gb = ub * ub * ir, gn = un * un * ir;
+    const double Gb = bk[0] * gb, Gn = nk[0] * gn;
+    const double g = fma(hk[0], gh, Gb + Gn);
+    const double k = fma(hk[0] * ir2 * ir2, r * uh2 - 3.0 * t,
+                         -ir * (Gb * (2.0 * ub + ir) + Gn * (2.0 * un + ir)));
+    const double xw = x * w[0] + y * w[1] + z * w[2];
+    const double kx = k * xw;
+    Hw[0] = g * w[0] + kx * x;
+    Hw[1] = g * w[1] + kx * y;
+    Hw[2] = g * w[2] + kx * z;
+    th[3] -= gh * xw;
+    th[4] += hk[0] * hk[2] * (uh2 * ir * xw);
+    th[6] -= gb * xw;
+    th[7] += 2.0 * Gb * ub * xw;
+    th[9] -= gn * xw;
+    th[10] += 2.0 * Gn * un * xw;
+    mn_adjoint(dk[0], dk[1], dk[7], x, y, z, w, Hw, th);
+  }
+};
 
 // ------------------------------------------------ potential and Hessian
 // (not on the integration hot path: each component in the inertial frame)

@@ -288,6 +288,34 @@ __device__ __forceinline__ void rk_end_stage(const DPot& P, double dir,
 }
 
 
+// A compile-time table read where it is used, by scalar loads: through its
+// plain name the compiler either folds the coefficients into code (two moves
+// for each) or hoists all their loads out of the enclosing loops and spills
+// the scalar registers to vector lanes, two lane reads for each use.  The
+// empty asm makes the address unknown at its place, so that the loads stay
+// after it; address space 4 (constant) makes them scalar.
+typedef const __attribute__((address_space(4))) double ConstDouble;
+__device__ __forceinline__ ConstDouble* table_here(const double* t) {
+  asm volatile("" : "+s"(t));
+  return (ConstDouble*)t;
+}
+
+// a x + c with c in scalar registers (from the plain expression the compiler
+// makes an accumulating FMA and copies c to vector registers first).
+__device__ __forceinline__ double fma_s(double a, double x, double c) {
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(x), "s"(c));
+  return r;
+}
+
+template <int D>
+__device__ __forceinline__ double horner_here(ConstDouble* c, double x) {
+  double acc = c[0];
+#pragma unroll
+  for (int d = 1; d < D; ++d) acc = fma_s(acc, x, c[d]);
+  return acc;
+}
+
 template <int D>
 __device__ __forceinline__ double horner(const double (&c)[D], double x) {
   double acc = c[0];

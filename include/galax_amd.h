@@ -356,7 +356,8 @@ int gx_integrate_shared(const gx_pot* pot, const gx_solver_cfg* cfg,
  * r_s).  Supported potentials: the Milky Way composition (Miyamoto-Nagai,
  * NFW, Hernquist, Hernquist, untranslated) and any single untranslated
  * Kepler/Hernquist/Miyamoto-Nagai/NFW/Plummer component; ntheta <= 12.
- * State is checkpointed every K steps; max_steps bounds the steps of any
+ * State is checkpointed every K steps, or at every step where that takes
+ * at most 4 GiB; max_steps bounds the steps of any
  * orbit (it sizes the workspace, gx_adjoint_workspace_bytes(n, max_steps,
  * K) bytes, 256-byte aligned).  status[n] (optional) is GX_SUCCESS or
  * GX_MAX_STEPS_REACHED.  Replaces differentiating evaluate_orbit /

@@ -101,3 +101,37 @@ def test_adjoint_single_component_kinds():
                   - _loss_oracle(mk(pm), solver, w0, 0.0, 80.0, None, 0.5, C)) / (2 * h)
             got = raw[j] * (G if j == 0 else 1.0)  # table slot 0 is G m
             assert got == pytest.approx(fd, rel=1e-5), (name, j)
+
+
+@pytest.mark.gpu
+def test_adjoint_does_not_depend_on_the_batch():
+    """An orbit's gradients are the same bits in batches of any size: ragged
+    workgroups, and a batch whose states exceed the memory kept for every
+    step, which is reversed by checkpointed segments instead."""
+    import torch
+
+    from galax_amd import _lib
+    from galax_amd.adjoint import adjoint_orbits
+
+    pot = gp.MilkyWayPotential()
+    n, steps, K = 160_037, 490, 64
+    lib = _lib.lib()
+    assert int(lib.gx_adjoint_workspace_bytes(n, steps, K)) < 56 * n * steps  # checkpointed
+    assert int(lib.gx_adjoint_workspace_bytes(1000, steps, K)) >= 56 * 1000 * steps  # every step
+    rng = np.random.default_rng(8)
+    w0 = np.tile(workloads.disk_ics(1600, 31), (101, 1))[:n]
+    t0 = -rng.uniform(1.0, 488.0, n)
+    ts = np.stack([0.37 * t0, np.zeros(n)], 1)  # inside a step, and its end
+    cot = rng.normal(size=(n, 2, 6))
+
+    def run(sel):
+        print(f"[case] adjoint batch {sel}", flush=True)
+        wb, raw, st = adjoint_orbits(pot, w0[sel], t0[sel], 0.0, torch.as_tensor(cot[sel]), dt0=1.0, ts=ts[sel],
+                                     ntheta=12, max_steps=steps, K=K)
+        assert int(st.abs().sum()) == 0
+        return wb.cpu().numpy(), raw.cpu().numpy()
+
+    big = run(slice(0, n))
+    for a, b in ((0, 1), (0, 64), (5, 70), (100, 227), (300, 428), (500, 629), (n - 300, n)):
+        for x, y in zip(run(slice(a, b)), big):
+            np.testing.assert_array_equal(x, y[a:b])

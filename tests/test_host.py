@@ -211,7 +211,7 @@ def test_numpy_gradient_matches_oracle():
 def _kernel_resources(tmp_path):
     """Kernel metadata (VGPRs, spills, scratch) of every kernel in the built
     library's gfx950 code objects: the .hip_fatbin section holds one offload
-    bundle per source file."""
+    bundle per source file (left as b<i>.o in tmp_path)."""
     tools = Path("/opt/rocm/llvm/bin")
     need = [tools / "llvm-objcopy", tools / "clang-offload-bundler", tools / "llvm-readelf"]
     if not _lib.LIB_PATH.exists() or not all(t.exists() for t in need):
@@ -260,6 +260,44 @@ def test_integrator_kernels_keep_their_occupancy(tmp_path):
                 assert spill <= max_spill, (n, spill)
             if not scratch_ok:
                 assert scratch == 0, (n, scratch)
+
+
+def test_no_spill_before_the_execution_mask_is_restored(tmp_path):
+    """Where divergent lanes meet again, a block opens by restoring the
+    execution mask.  Spill code that the compiler puts before that restore
+    runs for some lanes only and loses the others' values (seen once, in an
+    adjoint kernel built with spills): no kernel of the library has any."""
+    res = _kernel_resources(tmp_path)
+    objdump = Path("/opt/rocm/llvm/bin/llvm-objdump")
+    if not objdump.exists():
+        pytest.skip("llvm-objdump missing")
+    spill = re.compile(r"(scratch_|v_accvgpr_)")
+    bad, kernels = [], 0
+    for dev in sorted(tmp_path.glob("b*.o")):
+        asm = subprocess.run([str(objdump), "-d", "--no-show-raw-insn", "--symbolize-operands", str(dev)], check=True,
+                             capture_output=True, text=True).stdout
+        name, pending = "", None
+        for line in asm.splitlines():
+            head = re.match(r"^[0-9a-f]* ?<(\S+)>:", line)
+            if head:
+                if not head.group(1).startswith("L"):
+                    name = head.group(1)
+                    kernels += name in res
+                pending = []
+                continue
+            ins = line.split("//")[0].strip()
+            if not ins or pending is None:
+                continue
+            if spill.match(ins):
+                pending.append(ins)
+            elif ins.startswith("s_or_b64 exec, exec"):
+                if pending:
+                    bad.append((name, pending))
+                pending = None
+            elif not ins.startswith(("v_mov_b", "s_")) or ins.startswith(("s_cbranch", "s_branch", "s_endpgm")):
+                pending = None
+    assert kernels == len(res)
+    assert not bad, bad
 
 
 def test_caller_buffers_are_checked():
