@@ -695,6 +695,15 @@ int gx_potential_create(const gx_component* comps, int32_t ncomp,
       comps[1].kind == GX_NFW && comps[2].kind == GX_HERNQUIST &&
       comps[3].kind == GX_HERNQUIST)
     h->sig = kSigMilkyWay;
+  if (ncomp >= 4)
+    for (int m = 0; m < 3; ++m) {
+      h->dev.mw.disk[m] = dc[0].p[m];
+      h->dev.mw.halo[m] = dc[1].p[m];
+      if (m < 2) {
+        h->dev.mw.bulge[m] = dc[2].p[m];
+        h->dev.mw.nucleus[m] = dc[3].p[m];
+      }
+    }
   bool mw_origin = ncomp == 5;
   for (int i = 0; mw_origin && i < 4; ++i) mw_origin = comps[i].frame == GX_FRAME_NONE;
   if (mw_origin && comps[0].kind == GX_MIYAMOTO_NAGAI && comps[1].kind == GX_NFW &&

@@ -90,6 +90,11 @@ struct DTrack {
   long long lds_doubles;  // pieces + cells, when ncell > 0
 };
 
+// What EvalMW reads of its four rows (as in DComp::p).
+struct MwRows {
+  double disk[3], halo[3], bulge[2], nucleus[2];
+};
+
 struct DPot {
   const DComp* comps;
   const DTrack* tracks;
@@ -106,6 +111,8 @@ struct DPot {
   // load.
   DTrack trk;
   double kp[2];
+  // likewise the Milky Way rows (0-3) of the tables that start with them
+  MwRows mw;
 };
 
 // ------------------------------------------------------------- tracks
@@ -913,10 +920,10 @@ struct EvalMW {
                                              double z, double /*t*/,
                                              double& ax, double& ay,
                                              double& az) {
-    const double* dk = P.comps[0].p;
-    const double* hk = P.comps[1].p;
-    const double* bk = P.comps[2].p;
-    const double* nk = P.comps[3].p;
+    const double* dk = P.mw.disk;
+    const double* hk = P.mw.halo;
+    const double* bk = P.mw.bulge;
+    const double* nk = P.mw.nucleus;
     const double r2 = x * x + y * y + z * z;
     const double ir = rsqrt_fast(r2 + kTiny);
     const double r = (r2 + kTiny) * ir;

@@ -293,7 +293,10 @@ __device__ __forceinline__ void rk_end_stage(const DPot& P, double dir,
 // for each) or hoists all their loads out of the enclosing loops and spills
 // the scalar registers to vector lanes, two lane reads for each use.  The
 // empty asm makes the address unknown at its place, so that the loads stay
-// after it; address space 4 (constant) makes them scalar.
+// after it; address space 4 (constant) makes them scalar.  The dense output
+// of a step takes 316 instructions this way instead of 483 (1,048,576 orbits
+// of 300 Myr with 64 saves: 11.1 -> 9.9 ms, together with the Milky Way's rows
+// in the kernel arguments).
 typedef const __attribute__((address_space(4))) double ConstDouble;
 __device__ __forceinline__ ConstDouble* table_here(const double* t) {
   asm volatile("" : "+s"(t));
@@ -316,50 +319,61 @@ __device__ __forceinline__ double horner_here(ConstDouble* c, double x) {
   return acc;
 }
 
-template <int D>
-__device__ __forceinline__ double horner(const double (&c)[D], double x) {
-  double acc = c[0];
-#pragma unroll
-  for (int d = 1; d < D; ++d) acc = fma(acc, x, c[d]);
-  return acc;
-}
-
 // The dense output of a step (q, p at its start, step h, stage
 // accelerations g[0..SF-1] including the end stage) at th in [0, 1]:
-// diffrax's interpolant for the method, in Runge-Kutta-Nystrom form.
-// (The coefficient rows go to horner() by reference: the compiler then
-// loads them from the constant table into scalar registers once, which
-// measured lighter on the register file than folding them into the code.)
+// diffrax's interpolant for the method, in Runge-Kutta-Nystrom form.  The
+// weighted sums over the stages, one stage at a time, and the result.
+struct DenseSum {
+  double sq[3] = {0.0, 0.0, 0.0}, sp[3] = {0.0, 0.0, 0.0};
+
+  template <class M, int L>
+  __device__ __forceinline__ void add(ConstDouble* tq, ConstDouble* tp, double th,
+                                      const double (&g)[3]) {
+    constexpr int D = sizeof(M::dn.wq[0]) / sizeof(double);
+    if constexpr (M::dn.nq[L]) {
+      const double w = horner_here<D>(tq + D * L, th);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) sq[m] = fma(w, g[m], sq[m]);
+    }
+    if constexpr (M::dn.np[L]) {
+      const double w = horner_here<D>(tp + D * L, th);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) sp[m] = fma(w, g[m], sp[m]);
+    }
+  }
+  __device__ __forceinline__ void result(double th, double h, const double (&q)[3],
+                                         const double (&p)[3], double (&qo)[3],
+                                         double (&po)[3]) const {
+    const double ht = h * th, hht = h * ht;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      po[m] = fma(ht, sp[m], p[m]);
+      qo[m] = fma(hht, sq[m], fma(ht, p[m], q[m]));
+    }
+  }
+};
+
+template <int A, int B, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (A < B) {
+    f(std::integral_constant<int, A>{});
+    static_for<A + 1, B>(f);
+  }
+}
+
 template <class M>
 __device__ __forceinline__ void dense_eval(double th, double h,
                                            const double (&q)[3],
                                            const double (&p)[3],
                                            const double (&g)[M::SF][3],
                                            double (&qo)[3], double (&po)[3]) {
-  constexpr int SF = M::SF;
-  double sq0 = 0.0, sq1 = 0.0, sq2 = 0.0, sp0 = 0.0, sp1 = 0.0, sp2 = 0.0;
-#pragma unroll
-  for (int l = 0; l < SF; ++l) {
-    if (M::dn.nq[l]) {
-      const double w = horner(M::dn.wq[l], th);
-      sq0 = fma(w, g[l][0], sq0);
-      sq1 = fma(w, g[l][1], sq1);
-      sq2 = fma(w, g[l][2], sq2);
-    }
-    if (M::dn.np[l]) {
-      const double w = horner(M::dn.wp[l], th);
-      sp0 = fma(w, g[l][0], sp0);
-      sp1 = fma(w, g[l][1], sp1);
-      sp2 = fma(w, g[l][2], sp2);
-    }
-  }
-  const double ht = h * th, hht = h * ht;
-  po[0] = fma(ht, sp0, p[0]);
-  po[1] = fma(ht, sp1, p[1]);
-  po[2] = fma(ht, sp2, p[2]);
-  qo[0] = fma(hht, sq0, fma(ht, p[0], q[0]));
-  qo[1] = fma(hht, sq1, fma(ht, p[1], q[1]));
-  qo[2] = fma(hht, sq2, fma(ht, p[2], q[2]));
+  ConstDouble* tq = table_here(&M::dn.wq[0][0]);
+  ConstDouble* tp = table_here(&M::dn.wp[0][0]);
+  DenseSum s;
+  static_for<0, M::SF>([&](auto l) {
+    s.template add<M, decltype(l)::value>(tq, tp, th, g[decltype(l)::value]);
+  });
+  s.result(th, h, q, p, qo, po);
 }
 
 // One accepted step's dense-output record, in physical variables: start
