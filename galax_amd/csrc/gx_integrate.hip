@@ -26,6 +26,8 @@
 //     (diffrax's SaveAt(ts) interpolant), not by further field evaluations;
 //   * integration backwards in time runs in tau = -t with the velocity sign
 //     flipped, as diffrax does.
+// In the Milky Way fields, batches too small to fill the device go to teams
+// of four waves that share 64 orbits' steps (gx_team.hpp; launch_team's rule).
 // The controller follows diffrax 0.7.0's PIDController (error_order = method
 // order, RMS norm, factormin applied to rejected steps only), its automatic
 // initial step and its clip-to-end rule.
@@ -34,39 +36,11 @@
 
 #include "gx_internal.hpp"
 #include "gx_rk.hpp"
+#include "gx_steps.hpp"
+#include "gx_team.hpp"
 
 namespace gx {
 namespace {
-
-struct IArgs {
-  double dt0, rtol, atol, safety, factormin, factormax, dtmin, dtmax;
-  double c1, c2, c3;  // PID exponents (i+p+d)/k, -(p+2d)/k, d/k
-  long long max_steps;
-  int force_dtmin;
-  int t_stride;
-  int T;
-  int ts_mode;
-  int root8;  // c1 == 1/8 and c2 == c3 == 0: factor from three square roots
-  const double* w0;
-  const double* t0;
-  const double* t1;
-  const double* ts;
-  long long n;
-  const long long* order;
-  double* out;
-  int* status;
-  long long* nsteps;
-  long long* naccept;
-  unsigned long long* counter;
-  double* h0;  // first step per orbit, from the prepass (workspace)
-  double* a0;  // start acceleration per orbit [n][3], from the prepass
-  long long head_lanes;  // lanes that start on a fixed ticket
-  int head_only_once;    // head lanes take no second ticket
-  int chunk;             // tickets taken from the queue at a time
-  double* rec;           // dense records [n][rec_cap][kDenseRec] (dense mode)
-  long long rec_cap;
-  long long* nrec;       // records written per orbit
-};
 
 constexpr int kBlock = 256;
 constexpr long long kStepCap = 10000000;  // attempted steps per orbit
@@ -159,47 +133,6 @@ __device__ double start_orbit(const DPot& P, const IArgs& A, double dir,
     }
   }
   return h;
-}
-
-__device__ __forceinline__ double clip_to_end(double tprev, double tnext,
-                                              double t1, bool keep) {
-  return (tnext > t1 - 1e-10) ? (keep ? t1 : tprev + 0.5 * (t1 - tprev))
-                              : tnext;
-}
-
-__device__ __forceinline__ double save_time(const IArgs& A, long long orb,
-                                            int s, double t0, double t1) {
-  switch (A.ts_mode) {
-    case GX_TS_SHARED:
-      return A.ts[s];
-    case GX_TS_PER_ORBIT:
-      return A.ts[orb * A.T + s];
-    case GX_TS_LINSPACE:
-      return (s == A.T - 1) ? t1 : t0 + s * ((t1 - t0) / (A.T - 1));
-    default:
-      return t1;
-  }
-}
-
-__device__ __forceinline__ void write_save(const IArgs& A, long long orb,
-                                           int s, double dir,
-                                           const double (&q)[3],
-                                           const double (&p)[3]) {
-  double* o = A.out + (orb * A.T + s) * 6;
-  o[0] = q[0];
-  o[1] = q[1];
-  o[2] = q[2];
-  o[3] = dir * p[0];
-  o[4] = dir * p[1];
-  o[5] = dir * p[2];
-}
-
-__device__ __forceinline__ long long ticket_to_orbit(const IArgs& A,
-                                                     long long idx) {
-  if (idx >= A.n) return -1;
-  if (!A.order) return idx;
-  const long long o = A.order[idx];
-  return (o >= 0 && o < A.n) ? o : -1;  // the host validates permutations
 }
 
 // Start-of-orbit prepass for the evaluators that do not compute it inline:
@@ -366,62 +299,10 @@ __global__ void __launch_bounds__(kBlock)
           C.st[L] = GX_NONFINITE;
           done = true;
         } else {
-          bool keep = true;
           double next_t1;
-          if (PID) {
-            // diffrax's RMS norm of the scaled error, here through its
-            // mean square ms (the norm is below 1 exactly when ms is);
-            // quotients and roots by the short primitives, within about
-            // an ulp of the correctly rounded operations
-            double sq = 0.0;
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-              const double uq =
-                  eq[m] * rcp(A.atol + fmax(fabs(q[m]), fabs(q1[m])) * A.rtol);
-              const double up =
-                  ep[m] * rcp(A.atol + fmax(fabs(p[m]), fabs(p1[m])) * A.rtol);
-              sq += uq * uq + up * up;
-            }
-            const double ms = div6(sq);
-            keep = ms < 1.0;
-            const bool at_dtmin = C.at_dtmin[L] != 0;
-            if (A.dtmin > 0.0) keep = keep || at_dtmin;
-            // inv = 1 / norm = ms^(-1/2); zero (and subnormal) ms gives
-            // +inf, infinite ms 0, NaN stays NaN
-            const bool normal = ms >= kMinNormal && ms <= kMaxFinite;
-            const double special = (ms < kMinNormal)   ? __builtin_inf()
-                                   : (ms > kMaxFinite) ? 0.0
-                                                       : ms;
-            const double a = rsqrt_fast(ms);
-            const double inv = normal ? a : special;
-            double f;
-            if (A.root8) {
-              // inv^(1/8) = 1 / rsqrt(rsqrt(rsqrt(inv)))
-              f = normal ? rcp(rsqrt_fast(rsqrt_fast(rsqrt_fast(a)))) : special;
-            } else {
-              f = (A.c1 == 0.0) ? 1.0 : pow(inv, A.c1);
-              if (A.c2 != 0.0) f *= pow(C.prev_inv[L], A.c2);
-              if (A.c3 != 0.0) f *= pow(C.prev_prev_inv[L], A.c3);
-            }
-            const double fmin_ = keep ? 1.0 : A.factormin;
-            const double factor =
-                fmin(fmax(A.safety * f, fmin_), A.factormax);
-            double dt = fmin(h * factor, A.dtmax);
-            if (A.dtmin > 0.0) {
-              if (!A.force_dtmin && dt < A.dtmin)
-                C.st[L] = GX_DT_MIN_REACHED;
-              C.at_dtmin[L] = dt <= A.dtmin ? 1 : 0;
-              dt = fmax(dt, A.dtmin);
-            }
-            if (keep) {
-              // a zero or infinite error does not steer later steps
-              C.prev_prev_inv[L] = C.prev_inv[L];
-              C.prev_inv[L] = (inv == 0.0 || isinf(inv)) ? 1.0 : inv;
-            }
-            next_t1 = (keep ? tnext : tau) + dt;
-          } else {
-            next_t1 = tnext + A.dt0;
-          }
+          const bool keep = control_step<PID>(
+              A, tau, tnext, q, p, q1, p1, eq, ep, C.prev_inv[L],
+              C.prev_prev_inv[L], C.at_dtmin[L], C.st[L], next_t1);
           if (keep) {
             rk_end_stage<M, E>(P, dir, tnext, q1, g);
             // save times in (tau, tnext]: the step's end, or its dense
@@ -492,8 +373,76 @@ __global__ void k_reset_queue(unsigned long long* c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0ULL;
 }
 
+template <int ORDER, bool PID, class E>
+void launch_first_step(const gx_pot* pot, const IArgs& A, hipStream_t stream) {
+  long long fblocks = (A.n + 255) / 256;
+  const long long fcap = (long long)num_cus(pot->device) * 8;
+  if (fblocks > fcap) fblocks = fcap;
+  hipLaunchKernelGGL((k_first_step<ORDER, PID, E>), dim3((unsigned)fblocks), dim3(256), 0, stream,
+                     pot->dev, A);
+}
+
+// Evaluators with an integrator by teams of waves (gx_team.hpp).
+template <class M, class E>
+constexpr bool has_team = std::is_same_v<M, Dopri8> &&
+                          (std::is_same_v<E, EvalMilkyWay> || std::is_same_v<E, EvalMilkyWayPieces>);
+
+// Teams for batches that are bound by the latency of single orbits: GX_OK when
+// launched, kNoTeam when the batch does not suit.  The device holds 32,768
+// orbits in teams (two workgroups a CU) and 131,072 with a wave to 64 of them,
+// which is the faster form once the device is full.  Milliseconds with one
+// wave / with teams, PID, 300 Myr, in the Milky Way and on a staged track:
+//   orbits    final state   64 saves     | track: final   32 saves
+//    1,024     1.34  0.67   1.77  0.90   |  0.43  0.27   0.51  0.37
+//   32,768     1.58  1.00   1.97  1.24   |  2.33  1.45   2.22  1.76
+//   65,536     1.62  1.35   1.93  1.95   |  2.23  1.79   2.65  2.36
+//  131,072     2.27  2.02   2.68  3.21   |  2.44  2.13   2.84  3.02 (100,000)
+//  262,144     3.30  3.40   3.68  5.81
+// so the line is at 256 orbits a CU for one common span.  Spans of their own
+// leave the longest orbits at work after the rest: 131,072 orbits of 0.1 to
+// 5 Gyr with 64 saves take 46 / 27 ms, the 100,000 particles of a stream of
+// 4 Gyr 24.9 / 15.4 ms, and the line is at 512.
+constexpr int kNoTeam = 1;
+template <bool PID, class E, bool DENSE>
+int launch_team(const gx_pot* pot, IArgs& A, hipStream_t stream) {
+  const auto kern = k_team<PID, E, DENSE>;
+  const LaunchShape& ls = launch_shape();
+  const long long cus = num_cus(pot->device);
+  if (A.n > cus * (A.t_stride ? 512 : 256) / ls.parts) return kNoTeam;
+  size_t dyn = 0;
+  if constexpr (lds_track<E>::value) {
+    dyn = sizeof(double) * (size_t)pot->dev.trk.lds_doubles;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) != hipSuccess) {
+      (void)hipGetLastError();
+      return kNoTeam;
+    }
+  }
+  int occ = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, 256, dyn) != hipSuccess || occ < 1) {
+    (void)hipGetLastError();
+    return kNoTeam;  // a track too large beside the team's own LDS
+  }
+  long long blocks = cus * occ / ls.parts;
+  const long long need = (A.n + kTeamOrbits - 1) / kTeamOrbits;
+  if (blocks > need) blocks = need;
+  if (blocks < 1) blocks = 1;
+  const long long head = ls.head_lanes, lanes = blocks * kTeamOrbits;
+  A.head_lanes = head < lanes ? head : lanes;
+  A.head_only_once = (head > 0 && lanes >= 4 * head) ? 1 : 0;
+  A.chunk = ls.chunk;
+  hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, A.counter);
+  launch_first_step<8, PID, E>(pot, A, stream);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), dyn, stream, pot->dev, A);
+  return check(hipGetLastError());
+}
+
 template <class M, bool PID, class E, bool DENSE = false>
 int launch(const gx_pot* pot, IArgs& A, hipStream_t stream) {
+  if constexpr (has_team<M, E>) {
+    const int rc = launch_team<PID, E, DENSE>(pot, A, stream);
+    if (rc != kNoTeam) return rc;
+  }
   const auto kern = k_integrate<M, PID, E, DENSE>;
   const LaunchShape& ls = launch_shape();
   const int block = kBlock;
@@ -526,14 +475,7 @@ int launch(const gx_pot* pot, IArgs& A, hipStream_t stream) {
   A.head_only_once = (head > 0 && blocks * block >= 4 * head) ? 1 : 0;
   A.chunk = ls.chunk;
   hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, A.counter);
-  if constexpr (!E::kInlineFirstStep) {
-    long long fblocks = (A.n + 255) / 256;
-    const long long fcap = (long long)num_cus(pot->device) * 8;
-    if (fblocks > fcap) fblocks = fcap;
-    hipLaunchKernelGGL((k_first_step<M::order, PID, E>),
-                       dim3((unsigned)fblocks), dim3(256), 0, stream, pot->dev,
-                       A);
-  }
+  if constexpr (!E::kInlineFirstStep) launch_first_step<M::order, PID, E>(pot, A, stream);
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(block), dyn, stream,
                      pot->dev, A);
   return check(hipGetLastError());

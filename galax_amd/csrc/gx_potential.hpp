@@ -1027,6 +1027,24 @@ struct EvalMilkyWayTracked {
     ay -= g * Y;
     az -= g * Z;
   }
+  // The Plummer sphere at (dx, dy, dz) alone, for callers that evaluate the
+  // host apart from it.  acc_at's sum x^2 + y^2 is left to the compiler, which
+  // rounds y^2 first, except in a step's first stage (YFIRST = false), where
+  // it rounds x^2; written out here, so that both callers' bits agree.
+  template <bool YFIRST>
+  __device__ __forceinline__ static void add_tracked(const DPot& P, double x,
+                                                     double y, double z,
+                                                     double dx, double dy,
+                                                     double dz, double& ax,
+                                                     double& ay, double& az) {
+    const double X = x - dx, Y = y - dy, Z = z - dz;
+    const double R2 = YFIRST ? fma(X, X, Y * Y) : fma(Y, Y, X * X);
+    const double id = rsqrt_fast(fma(Z, Z, R2) + P.kp[1]);
+    const double g = P.kp[0] * id * id * id;
+    ax -= g * X;
+    ay -= g * Y;
+    az -= g * Z;
+  }
   __device__ __forceinline__ static void acc(const DPot& P, double x, double y,
                                              double z, double t, double& ax,
                                              double& ay, double& az) {
