@@ -573,6 +573,8 @@ int gx_potential_create(const gx_component* comps, int32_t ncomp,
     }
     dc[i].flags |= kGroupStart;
     dc[j - 1].flags |= kGroupEnd;
+    for (int k = j - 1, run = 0; k >= i; --k)
+      dc[k].track = run = comps[k].kind == GX_PLUMMER ? run + 1 : 0;
     i = j;
   }
   // tracks: validate knots; build dense-solution tracks

