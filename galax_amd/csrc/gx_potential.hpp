@@ -1035,6 +1035,12 @@ struct EvalMilkyWayRotating {
                                              double z, double t, double& ax,
                                              double& ay, double& az) {
     EvalMW::acc(P, x, y, z, t, ax, ay, az);
+    add_group(P, x, y, z, t, ax, ay, az);
+  }
+  __device__ __forceinline__ static void add_group(const DPot& P, double x,
+                                                   double y, double z, double t,
+                                                   double& ax, double& ay,
+                                                   double& az) {
     double s, c;
     sincos(comps_here(P)[4].f[3] * t, &s, &c);
     const double xr = x * c + y * s, yr = y * c - x * s;
@@ -1764,6 +1770,44 @@ __device__ inline double potential(const DPot& P, double x, double y,
     s += phi_model(c, P.aux, x - dx, y - dy, z - dz, t);
   }
   return s;
+}
+
+// The Milky Way model's Hessian in closed form: the spherical components' sum
+// as g I + K n n^T (n = x / r), the disk's as in mn_adjoint.
+__device__ __forceinline__ void mw_hessian(const DPot& P, double x, double y, double z, double* H) {
+  const double* dk = P.mw.disk;
+  const double* hk = P.mw.halo;
+  const double* bk = P.mw.bulge;
+  const double* nk = P.mw.nucleus;
+  const double R2 = x * x + y * y;
+  const double r2 = R2 + z * z;
+  // corrected roots and their reciprocals: a cubed rsqrt's error is three
+  // times its own
+  const double r = sqrt_fast(r2), ir = rcp(r);
+  const double uh = rcp(r + hk[1]), ub = rcp(r + bk[1]), un = rcp(r + nk[1]);
+  const double t = log1p_fast(r * hk[2]) * ir - uh;
+  const double G = hk[0] * ir * ir;
+  const double Gb = bk[0] * (ub * ub * ir), Gn = nk[0] * (un * un * ir);
+  const double g = fma(G, t, Gb + Gn);
+  const double K = G * (r * (uh * uh) - 3.0 * t) -
+                   (Gb * fma(2.0 * r, ub, 1.0) + Gn * fma(2.0 * r, un, 1.0));
+  const double S2 = z * z + dk[2];
+  const double S = sqrt_fast(S2), iS = rcp(S);
+  const double A = dk[1] + S;
+  const double iD = rcp(sqrt_fast(R2 + A * A));
+  const double t3 = dk[0] * (iD * iD * iD), t5 = 3.0 * t3;
+  const double zS = z * iS;
+  // unit vectors of the position and of the disk's (x, y, A z / S) / D
+  const double nx = x * ir, ny = y * ir, nz = z * ir;
+  const double vx = x * iD, vy = y * iD, vz = A * zS * iD;
+  const double d = g + t3;
+  const double Kx = K * nx, Ky = K * ny, wx = t5 * vx, wy = t5 * vy;
+  H[0] = fma(Kx, nx, d) - wx * vx;
+  H[4] = fma(Ky, ny, d) - wy * vy;
+  H[8] = fma(K * nz, nz, g) + fma(t3, zS * zS + A * iS * (dk[2] * (iS * iS)), -t5 * (vz * vz));
+  H[1] = H[3] = Kx * ny - wx * vy;
+  H[2] = H[6] = Kx * nz - wx * vz;
+  H[5] = H[7] = Ky * nz - wy * vz;
 }
 
 __device__ inline void hessian(const DPot& P, double x, double y, double z,
