@@ -37,6 +37,7 @@ SIGNATURES = {
     "gx_gradient": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i64, _vp, _vp]),
     "gx_potential_eval": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i64, _vp, _vp]),
     "gx_hessian": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i64, _vp, _vp]),
+    "gx_field_at": (ctypes.c_int, [_vp, _i32, _vp, _f64, _i64, _vp, _vp]),
     "gx_integrate_workspace_bytes": (_i64, [_i64]),
     "gx_integrate": (
         ctypes.c_int,

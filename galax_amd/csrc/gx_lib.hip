@@ -349,13 +349,24 @@ double group_rate(const gx_component& c) {
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
+// The times of a field call: t[n], one time in device memory, or by value
+// (t null).
+struct FieldTime {
+  const double* t;
+  int stride;
+  double value;
+  __device__ __forceinline__ double of(long long i) const {
+    return t ? t[stride ? i : 0] : value;
+  }
+};
+
 __global__ __launch_bounds__(kFieldBlock) void k_accel(
-    DPot P, const double* __restrict__ xyz, const double* __restrict__ t,
-    int t_stride, long long n, double* __restrict__ out, double sign) {
+    DPot P, const double* __restrict__ xyz, FieldTime t, long long n,
+    double* __restrict__ out, double sign) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += stride) {
-    const double ti = t[t_stride ? i : 0];
+    const double ti = t.of(i);
     double ax, ay, az;
     accel<true>(P, xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], ti, ax, ay,
                  az);
@@ -430,8 +441,8 @@ struct FieldHessian {
 
 template <class W, bool GROUP>
 __global__ __launch_bounds__(kFieldBlock) void k_field(
-    DPot P, const double* __restrict__ xyz, const double* __restrict__ t, int t_stride,
-    long long n, double* __restrict__ out, double sign) {
+    DPot P, const double* __restrict__ xyz, FieldTime t, long long n,
+    double* __restrict__ out, double sign) {
   __shared__ double s[W::kOut * kFieldBlock];
   const int tid = threadIdx.x;
   for (long long i0 = (long long)blockIdx.x * kFieldBlock; i0 < n;
@@ -442,7 +453,7 @@ __global__ __launch_bounds__(kFieldBlock) void k_field(
       const int j = k * kFieldBlock + tid;
       if (j < 3 * m) s[j] = xyz[3 * i0 + j];
     }
-    const double ti = tid < m ? t[t_stride ? i0 + tid : 0] : 0.0;
+    const double ti = tid < m ? t.of(i0 + tid) : 0.0;
     __syncthreads();
     double o[W::kOut];
     if (tid < m)
@@ -463,22 +474,22 @@ __global__ __launch_bounds__(kFieldBlock) void k_field(
 }
 
 template <class W, bool GROUP>
-int launch_field(const gx_pot* pot, const double* xyz, const double* t, int32_t t_stride,
-                 int64_t n, double* out, void* stream, double sign) {
+int launch_field(const gx_pot* pot, const double* xyz, FieldTime t, int64_t n, double* out,
+                 void* stream, double sign) {
   long long blocks = (n + kFieldBlock - 1) / kFieldBlock;
   if (blocks > (1 << 20)) blocks = 1 << 20;
   hipLaunchKernelGGL((k_field<W, GROUP>), dim3((unsigned)blocks), dim3(kFieldBlock), 0,
-                     (hipStream_t)stream, pot->dev, xyz, t, t_stride, (long long)n, out, sign);
+                     (hipStream_t)stream, pot->dev, xyz, t, (long long)n, out, sign);
   return check(hipGetLastError());
 }
 
 __global__ __launch_bounds__(kFieldBlock) void k_potential(
-    DPot P, const double* __restrict__ xyz, const double* __restrict__ t,
-    int t_stride, long long n, double* __restrict__ out) {
+    DPot P, const double* __restrict__ xyz, FieldTime t, long long n,
+    double* __restrict__ out) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += stride) {
-    const double ti = t[t_stride ? i : 0];
+    const double ti = t.of(i);
     out[i] = potential(P, xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], ti);
   }
 }
@@ -504,12 +515,12 @@ __global__ void k_math_check(const double* __restrict__ x, long long n,
 }
 
 __global__ __launch_bounds__(kFieldBlock) void k_hessian(
-    DPot P, const double* __restrict__ xyz, const double* __restrict__ t,
-    int t_stride, long long n, double* __restrict__ out) {
+    DPot P, const double* __restrict__ xyz, FieldTime t, long long n,
+    double* __restrict__ out) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += stride) {
-    const double ti = t[t_stride ? i : 0];
+    const double ti = t.of(i);
     double H[9];
     hessian(P, xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], ti, H);
     for (int k = 0; k < 9; ++k) out[9 * i + k] = H[k];
@@ -855,51 +866,76 @@ int gx_potential_destroy(gx_pot* pot) {
   return GX_OK;
 }
 
-static int launch_accel(const gx_pot* pot, const double* xyz, const double* t,
-                        int32_t t_stride, int64_t n, double* out, void* stream,
-                        double sign) {
-  int ok = field_args_ok(pot, xyz, t, t_stride, n, out);
-  if (ok != 1) return ok;
+static int launch_accel(const gx_pot* pot, const double* xyz, FieldTime t,
+                        int64_t n, double* out, void* stream, double sign) {
   if (pot->sig == kSigMilkyWay)
-    return launch_field<FieldAcc, false>(pot, xyz, t, t_stride, n, out, stream, sign);
+    return launch_field<FieldAcc, false>(pot, xyz, t, n, out, stream, sign);
   if (pot->sig == kSigMilkyWayRotating)
-    return launch_field<FieldAcc, true>(pot, xyz, t, t_stride, n, out, stream, sign);
+    return launch_field<FieldAcc, true>(pot, xyz, t, n, out, stream, sign);
   hipLaunchKernelGGL(k_accel, dim3(field_grid(pot, n)), dim3(kFieldBlock), 0,
-                     (hipStream_t)stream, pot->dev, xyz, t, t_stride,
-                     (long long)n, out, sign);
+                     (hipStream_t)stream, pot->dev, xyz, t, (long long)n, out,
+                     sign);
+  return check(hipGetLastError());
+}
+
+static int launch_potential(const gx_pot* pot, const double* xyz, FieldTime t,
+                            int64_t n, double* phi, void* stream) {
+  hipLaunchKernelGGL(k_potential, dim3(field_grid(pot, n)), dim3(kFieldBlock),
+                     0, (hipStream_t)stream, pot->dev, xyz, t, (long long)n,
+                     phi);
+  return check(hipGetLastError());
+}
+
+static int launch_hessian(const gx_pot* pot, const double* xyz, FieldTime t,
+                          int64_t n, double* hess, void* stream) {
+  if (pot->sig == kSigMilkyWay)
+    return launch_field<FieldHessian, false>(pot, xyz, t, n, hess, stream, 1.0);
+  hipLaunchKernelGGL(k_hessian, dim3(field_grid(pot, n)), dim3(kFieldBlock), 0,
+                     (hipStream_t)stream, pot->dev, xyz, t, (long long)n, hess);
   return check(hipGetLastError());
 }
 
 int gx_acceleration(const gx_pot* pot, const double* xyz, const double* t,
                     int32_t t_stride, int64_t n, double* acc, void* stream) {
-  return launch_accel(pot, xyz, t, t_stride, n, acc, stream, 1.0);
+  const int ok = field_args_ok(pot, xyz, t, t_stride, n, acc);
+  return ok != 1 ? ok : launch_accel(pot, xyz, {t, t_stride, 0.0}, n, acc, stream, 1.0);
 }
 
 int gx_gradient(const gx_pot* pot, const double* xyz, const double* t,
                 int32_t t_stride, int64_t n, double* grad, void* stream) {
-  return launch_accel(pot, xyz, t, t_stride, n, grad, stream, -1.0);
+  const int ok = field_args_ok(pot, xyz, t, t_stride, n, grad);
+  return ok != 1 ? ok : launch_accel(pot, xyz, {t, t_stride, 0.0}, n, grad, stream, -1.0);
 }
 
 int gx_potential_eval(const gx_pot* pot, const double* xyz, const double* t,
                       int32_t t_stride, int64_t n, double* phi, void* stream) {
-  int ok = field_args_ok(pot, xyz, t, t_stride, n, phi);
-  if (ok != 1) return ok;
-  hipLaunchKernelGGL(k_potential, dim3(field_grid(pot, n)), dim3(kFieldBlock),
-                     0, (hipStream_t)stream, pot->dev, xyz, t, t_stride,
-                     (long long)n, phi);
-  return check(hipGetLastError());
+  const int ok = field_args_ok(pot, xyz, t, t_stride, n, phi);
+  return ok != 1 ? ok : launch_potential(pot, xyz, {t, t_stride, 0.0}, n, phi, stream);
 }
 
 int gx_hessian(const gx_pot* pot, const double* xyz, const double* t,
                int32_t t_stride, int64_t n, double* hess, void* stream) {
-  int ok = field_args_ok(pot, xyz, t, t_stride, n, hess);
+  const int ok = field_args_ok(pot, xyz, t, t_stride, n, hess);
+  return ok != 1 ? ok : launch_hessian(pot, xyz, {t, t_stride, 0.0}, n, hess, stream);
+}
+
+int gx_field_at(const gx_pot* pot, int32_t what, const double* xyz, double t,
+                int64_t n, double* out, void* stream) {
+  const int ok = field_args_ok(pot, xyz, &t, 0, n, out);
   if (ok != 1) return ok;
-  if (pot->sig == kSigMilkyWay)
-    return launch_field<FieldHessian, false>(pot, xyz, t, t_stride, n, hess, stream, 1.0);
-  hipLaunchKernelGGL(k_hessian, dim3(field_grid(pot, n)), dim3(kFieldBlock), 0,
-                     (hipStream_t)stream, pot->dev, xyz, t, t_stride,
-                     (long long)n, hess);
-  return check(hipGetLastError());
+  const FieldTime at = {nullptr, 0, t};
+  switch (what) {
+    case GX_FIELD_ACCELERATION:
+      return launch_accel(pot, xyz, at, n, out, stream, 1.0);
+    case GX_FIELD_GRADIENT:
+      return launch_accel(pot, xyz, at, n, out, stream, -1.0);
+    case GX_FIELD_POTENTIAL:
+      return launch_potential(pot, xyz, at, n, out, stream);
+    case GX_FIELD_HESSIAN:
+      return launch_hessian(pot, xyz, at, n, out, stream);
+    default:
+      return GX_EINVAL;
+  }
 }
 
 int gx_set_launch_shape(int32_t block, int32_t blocks_per_cu,

@@ -197,6 +197,16 @@ int gx_potential_eval(const gx_pot* pot, const double* xyz, const double* t,
                       int32_t t_stride, int64_t n, double* phi, void* stream);
 int gx_hessian(const gx_pot* pot, const double* xyz, const double* t,
                int32_t t_stride, int64_t n, double* hess, void* stream);
+/* Any of them at one time given by value: a host scalar needs no device copy
+ * of its own (no separate reference entry point). */
+enum gx_field_what {
+  GX_FIELD_ACCELERATION = 0,
+  GX_FIELD_GRADIENT = 1,
+  GX_FIELD_POTENTIAL = 2,
+  GX_FIELD_HESSIAN = 3
+};
+int gx_field_at(const gx_pot* pot, int32_t what, const double* xyz, double t,
+                int64_t n, double* out, void* stream);
 
 /* ----------------------------------------------------------- integration */
 enum gx_method { GX_DOPRI8 = 0, GX_DOPRI5 = 1 };
