@@ -383,7 +383,7 @@ __global__ __launch_bounds__(kFieldBlock) void k_accel(
 // wave and needs the alignment of one double only.  Millions of points are
 // then bound by memory, thousands by the launch.  4,000,037 accelerations
 // (192 MB, 37 us at the rate of a copy): 134 -> 38 us; 1,000,000 Hessians: 84
-// -> 22 us; 1,000,000 accelerations with a group of 65 rows: 432 -> 74 us.
+// -> 34 us; 1,000,000 accelerations with a group of 65 rows: 432 -> 86 us.
 struct FieldAcc {
   static constexpr int kOut = 3;
   // accel()'s rows 0 .. 3 with their kinds at compile time, and the group
@@ -394,12 +394,14 @@ struct FieldAcc {
     const double ir = rsqrt_fast(r2 + kTiny), r = (r2 + kTiny) * ir;
     double ax = 0.0, ay = 0.0, az = 0.0;
     mn_acc(P.mw.disk, x, y, z, ax, ay, az);
-    const double g = sph_g(GX_NFW, P.mw.halo, r2, r, ir) +
-                     (sph_g(GX_HERNQUIST, P.mw.bulge, r2, r, ir) +
-                      sph_g(GX_HERNQUIST, P.mw.nucleus, r2, r, ir));
-    ax -= g * x;
-    ay -= g * y;
-    az -= g * z;
+    auto add = [&](double g) {
+      ax -= g * x;
+      ay -= g * y;
+      az -= g * z;
+    };
+    add(sph_g(GX_NFW, P.mw.halo, r2, r, ir));
+    add(sph_g(GX_HERNQUIST, P.mw.bulge, r2, r, ir));
+    add(sph_g(GX_HERNQUIST, P.mw.nucleus, r2, r, ir));
     if (GROUP) EvalMilkyWayRotating::add_group(P, x, y, z, t, ax, ay, az);
     o[0] = sign * ax;
     o[1] = sign * ay;
@@ -412,14 +414,9 @@ struct FieldHessian {
   template <bool GROUP>
   __device__ __forceinline__ static void at(const DPot& P, double x, double y, double z, double t,
                                             double, double* o) {
-    const double r2 = x * x + y * y + z * z, S2 = z * z + P.mw.disk[2];
-    if (r2 > 1e-8 && S2 > 1e-200 && r2 + S2 < 1e200) {
-      mw_hessian(P, x, y, z, o);
-      return;
-    }
-    // the centre, where the halo's differences cancel, and what overflows: as
-    // hessian(), row by row (one at a time, or this path's registers halve the
-    // waves of the other)
+    // hessian()'s rows with their kinds at compile time, to the bit (a stream's
+    // release points come from it), one at a time: unrolled they take 352
+    // registers, one wave a SIMD
 #pragma unroll
     for (int k = 0; k < 9; ++k) o[k] = 0.0;
 #pragma nounroll

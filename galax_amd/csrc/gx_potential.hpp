@@ -967,15 +967,15 @@ __device__ __forceinline__ double minus_rounded(double a, double b) {
   return a - b;
 }
 
-// A Plummer row's share of the group's sums at the co-rotating point.
-__device__ __forceinline__ void plummer_row(ConstComp& m, double xr, double yr, double z,
-                                            double (&a)[3]) {
-  const double dx = xr - m.f[0], dy = yr - m.f[1], dz = z - m.f[2];
-  const double id = rsqrt_fast(fma(dz, dz, fma(dx, dx, dy * dy)) + m.p[1]);
-  const double g = m.p[0] * id * id * id;
-  a[0] = g * dx;
-  a[1] = g * dy;
-  a[2] = g * dz;
+// A Plummer row's G m / d^3 at the co-rotating point, and the point relative
+// to it.
+__device__ __forceinline__ double plummer_row(ConstComp& m, double xr, double yr, double z,
+                                              double (&d)[3]) {
+  d[0] = xr - m.f[0];
+  d[1] = yr - m.f[1];
+  d[2] = z - m.f[2];
+  const double id = rsqrt_fast(fma(d[2], d[2], fma(d[0], d[0], d[1] * d[1])) + m.p[1]);
+  return m.p[0] * id * id * id;
 }
 
 // The group of perturbers (rows 4 .. n-1) at the co-rotating point, in the
@@ -1001,19 +1001,19 @@ __device__ __forceinline__ void group_acc(const DPot& P, double xr, double yr, d
       ++i;
     }
     for (; run >= 4; run -= 4, i += 4) {
-      double a[4][3];
+      double d[4][3], a[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) plummer_row(rows[i + j], xr, yr, z, a[j]);
+      for (int j = 0; j < 4; ++j) a[j] = plummer_row(rows[i + j], xr, yr, z, d[j]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a[j][m]);
+        for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a[j] * d[j][m]);
     }
     for (; run > 0; --run, ++i) {
-      double a[3];
-      plummer_row(rows[i], xr, yr, z, a);
+      double d[3];
+      const double a = plummer_row(rows[i], xr, yr, z, d);
 #pragma unroll
-      for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a[m]);
+      for (int m = 0; m < 3; ++m) g[m] = minus_rounded(g[m], a * d[m]);
     }
   }
   gx = g[0];
@@ -1625,6 +1625,9 @@ __device__ inline void hess_model(const DComp& c, const double* aux,
         d1 = GM * r * id * id * id;
         d2 = GM * (p[1] - 2.0 * rr) * id * id * id * id * id;
       }
+      // rounded here for every caller: where the kind is a constant the
+      // compiler fuses d2's product into the difference below
+      asm("" : "+v"(d1), "+v"(d2));
       const double g = d1 / r;
       const double k = (d2 - g) / rr;
       for (int a = 0; a < 3; ++a)
@@ -1634,7 +1637,7 @@ __device__ inline void hess_model(const DComp& c, const double* aux,
     }
     case GX_MIYAMOTO_NAGAI: {
       const double GM = p[0], b2 = p[2];
-      const double S2 = z * z + b2, S = sqrt(S2);
+      const double S2 = fma(z, z, b2), S = sqrt(S2);
       const double A = p[1] + S;
       const double D2 = x * x + y * y + A * A;
       const double D = sqrt(D2);
@@ -1770,44 +1773,6 @@ __device__ inline double potential(const DPot& P, double x, double y,
     s += phi_model(c, P.aux, x - dx, y - dy, z - dz, t);
   }
   return s;
-}
-
-// The Milky Way model's Hessian in closed form: the spherical components' sum
-// as g I + K n n^T (n = x / r), the disk's as in mn_adjoint.
-__device__ __forceinline__ void mw_hessian(const DPot& P, double x, double y, double z, double* H) {
-  const double* dk = P.mw.disk;
-  const double* hk = P.mw.halo;
-  const double* bk = P.mw.bulge;
-  const double* nk = P.mw.nucleus;
-  const double R2 = x * x + y * y;
-  const double r2 = R2 + z * z;
-  // corrected roots and their reciprocals: a cubed rsqrt's error is three
-  // times its own
-  const double r = sqrt_fast(r2), ir = rcp(r);
-  const double uh = rcp(r + hk[1]), ub = rcp(r + bk[1]), un = rcp(r + nk[1]);
-  const double t = log1p_fast(r * hk[2]) * ir - uh;
-  const double G = hk[0] * ir * ir;
-  const double Gb = bk[0] * (ub * ub * ir), Gn = nk[0] * (un * un * ir);
-  const double g = fma(G, t, Gb + Gn);
-  const double K = G * (r * (uh * uh) - 3.0 * t) -
-                   (Gb * fma(2.0 * r, ub, 1.0) + Gn * fma(2.0 * r, un, 1.0));
-  const double S2 = z * z + dk[2];
-  const double S = sqrt_fast(S2), iS = rcp(S);
-  const double A = dk[1] + S;
-  const double iD = rcp(sqrt_fast(R2 + A * A));
-  const double t3 = dk[0] * (iD * iD * iD), t5 = 3.0 * t3;
-  const double zS = z * iS;
-  // unit vectors of the position and of the disk's (x, y, A z / S) / D
-  const double nx = x * ir, ny = y * ir, nz = z * ir;
-  const double vx = x * iD, vy = y * iD, vz = A * zS * iD;
-  const double d = g + t3;
-  const double Kx = K * nx, Ky = K * ny, wx = t5 * vx, wy = t5 * vy;
-  H[0] = fma(Kx, nx, d) - wx * vx;
-  H[4] = fma(Ky, ny, d) - wy * vy;
-  H[8] = fma(K * nz, nz, g) + fma(t3, zS * zS + A * iS * (dk[2] * (iS * iS)), -t5 * (vz * vz));
-  H[1] = H[3] = Kx * ny - wx * vy;
-  H[2] = H[6] = Kx * nz - wx * vz;
-  H[5] = H[7] = Ky * nz - wy * vz;
 }
 
 __device__ inline void hessian(const DPot& P, double x, double y, double z,

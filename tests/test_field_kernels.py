@@ -1,6 +1,6 @@
 """The Milky Way's field kernels (alone and with a rotating group) at the edges
 of a workgroup, on positions of every alignment, with a time for all points or
-for each, and where the Hessian changes its form, against the oracle.
+for each, far out and at the centre, against the oracle.
 
 Bound: some 30 rounded operations a value, each within two units in the last
 place (7e-15), times the halo's cancellation between 0.05 and 60 kpc (below
