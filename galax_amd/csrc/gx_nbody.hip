@@ -22,6 +22,7 @@
 #include "gx_internal.hpp"
 #include "gx_potential.hpp"
 #include "gx_rk.hpp"
+#include "gx_slots.hpp"
 #include "gx_tableau.hpp"
 
 namespace gx {
@@ -392,9 +393,7 @@ __global__ void __launch_bounds__(kNbThreads) k_nbody(DPot P, NArgs A) {
 // A meeting costs more than the sums of 1,024 bodies, so it is one store and
 // one load through the level that all XCDs share, with no flag, no
 // read-modify-write and no cache flush: every published value is its own
-// flag.  Values are written and read by relaxed device-scope atomics of 64
-// bits; a slot holds kNbEmpty (a NaN that arithmetic does not produce) until
-// its owner has published, and a reader repeats its load while it sees that.
+// flag (gx_slots.hpp).
 // Three buffers take turns by meeting.  Having read meeting k - 1, an owner
 // knows that every workgroup has come to it and so has read meeting k - 2,
 // whose buffer is the one of meeting k + 1: it empties its own slots there,
@@ -410,39 +409,16 @@ constexpr int kNbWaves = kNbThreads / 64;
 constexpr int kNbOwnMax = 16;   // bodies of a workgroup when G > 1
 constexpr int kNbGroups = 256;  // most workgroups
 
-typedef unsigned long long NbSlot;
-constexpr NbSlot kNbEmpty = 0xfff8dead5a5a0001ull;
-constexpr NbSlot kNbNan = 0x7ff8000000000000ull;
-
 struct NGrid {
   int G;         // workgroups
   int own;       // bodies of a workgroup
-  NbSlot* pos;   // [3][3][n] published positions
-  NbSlot* part;  // [3][2][G] published error sums and non-finite counts
+  Slot* pos;   // [3][3][n] published positions
+  Slot* part;  // [3][2][G] published error sums and non-finite counts
 };
 
-__global__ void k_nb_empty(NbSlot* slots, long long m) {
+__global__ void k_nb_empty(Slot* slots, long long m) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < m) slots[i] = kNbEmpty;
-}
-
-__device__ __forceinline__ void put_slot(NbSlot* p, NbSlot v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void put_slot(NbSlot* p, double v) {
-  put_slot(p, v == v ? (NbSlot)__double_as_longlong(v) : kNbNan);
-}
-__device__ __forceinline__ NbSlot get_slot(const NbSlot* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// All G workgroups are resident and take the same decisions, so every one
-// publishes for every meeting and every wait ends.
-__device__ __forceinline__ double await_slot(const NbSlot* p, NbSlot seen) {
-  while (seen == kNbEmpty) {
-    __builtin_amdgcn_s_sleep(1);
-    seen = get_slot(p);
-  }
-  return __longlong_as_double((long long)seen);
+  if (i < m) slots[i] = kSlotEmpty;
 }
 
 // Dynamic LDS of a workgroup (doubles): all positions and masses, then the
@@ -502,7 +478,7 @@ struct NbGridSolve {
   // The workgroup's two sums for the coming meeting.
   __device__ __forceinline__ void offer(double a, double b) {
     if (X.G == 1 || tid != 0) return;
-    NbSlot* p = X.part + (size_t)turn * 2 * X.G + blockIdx.x;
+    Slot* p = X.part + (size_t)turn * 2 * X.G + blockIdx.x;
     put_slot(p, a);
     put_slot(p + X.G, b);
   }
@@ -510,9 +486,9 @@ struct NbGridSolve {
   // The meeting's sums over all workgroups.
   __device__ __forceinline__ void total(double& a, double& b) {
     if (X.G == 1) return;
-    const NbSlot* p = X.part + (size_t)turn * 2 * X.G + tid;
+    const Slot* p = X.part + (size_t)turn * 2 * X.G + tid;
     const bool in = tid < X.G;
-    const NbSlot va = in ? get_slot(p) : 0, vb = in ? get_slot(p + X.G) : 0;
+    const Slot va = in ? get_slot(p) : 0, vb = in ? get_slot(p + X.G) : 0;
     a = await_slot(p, va);
     b = await_slot(p + X.G, vb);
     sum(a, b);
@@ -523,8 +499,8 @@ struct NbGridSolve {
     if (X.G > 1 && tid < 64) {
       const int next = turn == 0 ? 2 : turn - 1;  // of the meeting after next
       if (tid < 3 * cnt)
-        put_slot(X.pos + ((size_t)next * 3 + tid / cnt) * n + first + tid % cnt, kNbEmpty);
-      if (tid < 2) put_slot(X.part + ((size_t)next * 2 + tid) * X.G + blockIdx.x, kNbEmpty);
+        put_slot(X.pos + ((size_t)next * 3 + tid / cnt) * n + first + tid % cnt, kSlotEmpty);
+      if (tid < 2) put_slot(X.part + ((size_t)next * 2 + tid) * X.G + blockIdx.x, kSlotEmpty);
     }
     turn = turn == 2 ? 0 : turn + 1;
   }
@@ -546,9 +522,9 @@ struct NbGridSolve {
   __device__ __forceinline__ void fetch() {
     if (X.G > 1) {
       constexpr int R = 6;  // loads in flight
-      const NbSlot* src = X.pos + (size_t)turn * 3 * n;
+      const Slot* src = X.pos + (size_t)turn * 3 * n;
       for (int k0 = tid; k0 < 3 * n; k0 += R * kNbThreads) {
-        NbSlot v[R];
+        Slot v[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           const int k = k0 + r * kNbThreads;
@@ -942,7 +918,7 @@ int launch_grid(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
   X.G = (int)((A.n + X.own - 1) / X.own);
   // what G workgroups exchange (72 bytes a body, 48 a workgroup) fits where
   // the one-workgroup kernel keeps its state (432 bytes a body)
-  X.pos = reinterpret_cast<NbSlot*>(static_cast<char*>(workspace) + 256);
+  X.pos = reinterpret_cast<Slot*>(static_cast<char*>(workspace) + 256);
   X.part = X.pos + 9 * A.n;
   const size_t lds = sizeof(double) * nb_lds_doubles(A.n, X.own, M::SF);
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),

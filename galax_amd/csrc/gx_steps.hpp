@@ -59,6 +59,12 @@ __device__ __forceinline__ double save_time(const IArgs& A, long long orb,
   }
 }
 
+__device__ __forceinline__ void orbit_span(const IArgs& A, long long orb, double& t0,
+                                           double& t1) {
+  t0 = A.t0[A.t_stride ? orb : 0];
+  t1 = A.t1[A.t_stride ? orb : 0];
+}
+
 __device__ __forceinline__ void write_save(const IArgs& A, long long orb,
                                            int s, double dir,
                                            const double (&q)[3],

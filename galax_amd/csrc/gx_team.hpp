@@ -265,13 +265,157 @@ struct TeamSums {
   }
 };
 
+// What the field and track waves need at the start of a step.
+template <bool TRACK>
+__device__ __forceinline__ void team_publish(TeamShared<TRACK>& S, int lane, double tau,
+                                             double tnext, double dir, const double (&q)[3],
+                                             const double (&p)[3]) {
+  constexpr auto& K = Dopri8::kf;
+  const double h = tnext - tau;
+  S.hh[lane] = h * h;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const double hp = h * p[m];
+    S.x1[0][m][lane] = fma(K.rs[1], hp, q[m]);
+    S.x1[1][m][lane] = fma(K.rs[2], hp, q[m]);
+  }
+  if constexpr (TRACK) {
+    S.when[0][lane] = tau;
+    S.when[1][lane] = h;
+    S.when[2][lane] = tnext;
+    S.when[3][lane] = dir;
+  }
+}
+
+// What the saving wave needs at its end (kept: the record's index + 1).
+__device__ __forceinline__ int record_slot(long long nacc, long long cap) {
+  return (int)(nacc <= cap ? nacc : cap + 1);
+}
+__device__ __forceinline__ void team_outcome(TeamShared<false>& S, int lane, bool keep, int kept,
+                                             bool done, double tend, const double (&q1)[3],
+                                             const double (&p1)[3]) {
+  S.kept[lane] = keep ? kept : 0;
+  S.done[lane] = done ? 1 : 0;
+  S.end[0][lane] = tend;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    S.end[1 + m][lane] = q1[m];
+    S.end[4 + m][lane] = p1[m];
+  }
+}
+
+template <bool TRACK>
+__device__ __forceinline__ void team_stage_acc(const TeamShared<TRACK>& S, int b, int l, int lane,
+                                               double (&g)[3]) {
+#pragma unroll
+  for (int m = 0; m < 3; ++m) g[m] = S.g[b][l][m][lane];
+}
+
+// Wave 2's sums from a step's start through its stage 12 (levels 1 to 6, a
+// barrier after each): the end state and the error estimate; false if the end
+// state is not finite.
+template <bool PID, bool TRACK>
+__device__ __forceinline__ bool team_rows(TeamShared<TRACK>& S, int b, int lane, double tau,
+                                          double h, const double (&q)[3], const double (&p)[3],
+                                          double (&q1)[3], double (&p1)[3], double (&eq)[3],
+                                          double (&ep)[3]) {
+  using M = Dopri8;
+  constexpr int SF = M::SF;
+  constexpr auto& K = M::kf;
+  const double hh = h * h;
+  const double hp[3] = {h * p[0], h * p[1], h * p[2]};
+  auto load = [&](int l, double (&g)[3]) { team_stage_acc(S, b, l, lane, g); };
+  TeamSums s;
+#pragma unroll
+  for (int i = 0; i < kTeamSums; ++i) s.row[i][0] = s.row[i][1] = s.row[i][2] = 0.0;
+  // the next level's rows, for its two stages
+  auto hand_over = [&](auto level) {
+    constexpr int lv = decltype(level)::value;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      constexpr int i0 = 2 * lv - 1;
+      if (i0 + w < SF) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+          S.x[lv & 1][w][m][lane] = fma(M::kf.rs[i0 + w < SF ? i0 + w : 0], hp[m], q[m]);
+          S.x[lv & 1][w][m + 3][lane] = s.row[i0 + w < SF ? i0 + w : 0][m];
+        }
+      }
+    }
+  };
+  auto add_two = [&](auto first, const double (&g1)[3], const double (&g2)[3]) {
+    constexpr int L = decltype(first)::value;
+    ConstDouble* w = table_here(TeamWeights::t.w + TeamWeights::t.first[L]);
+    s.add<L, L, PID>(w, g1);
+    s.add<L + 1, L, PID>(w, g2);
+  };
+  double ga[3], gb[3];
+  // level 1: the start acceleration
+  if (TRACK) __syncthreads();
+  team_start(S, b, lane, ga);
+#pragma unroll
+  for (int m = 0; m < 3; ++m) S.start[m][lane] = S.g[b][0][m][lane] = ga[m];
+  s.add<0, 0, PID>(table_here(TeamWeights::t.w), ga);
+  hand_over(std::integral_constant<int, 2>{});
+  __syncthreads();
+  // levels 2 .. 6: the stages of the level before
+  if constexpr (!TRACK) {
+    S.begin[0][lane] = tau;
+    S.begin[1][lane] = h;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      S.begin[2 + m][lane] = q[m];
+      S.begin[5 + m][lane] = p[m];
+    }
+  }
+  load(1, ga);
+  load(2, gb);
+  add_two(std::integral_constant<int, 1>{}, ga, gb);
+  hand_over(std::integral_constant<int, 3>{});
+  __syncthreads();
+  load(3, ga);
+  load(4, gb);
+  add_two(std::integral_constant<int, 3>{}, ga, gb);
+  hand_over(std::integral_constant<int, 4>{});
+  __syncthreads();
+  load(5, ga);
+  load(6, gb);
+  add_two(std::integral_constant<int, 5>{}, ga, gb);
+  hand_over(std::integral_constant<int, 5>{});
+  __syncthreads();
+  load(7, ga);
+  load(8, gb);
+  add_two(std::integral_constant<int, 7>{}, ga, gb);
+  hand_over(std::integral_constant<int, 6>{});
+  __syncthreads();
+  load(9, ga);
+  load(10, gb);
+  add_two(std::integral_constant<int, 9>{}, ga, gb);
+  hand_over(std::integral_constant<int, 7>{});
+  __syncthreads();
+  // level 7: the step's end, beside the end stage
+  load(11, ga);
+  load(12, gb);
+  add_two(std::integral_constant<int, 11>{}, ga, gb);
+  bool finite = true;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const double a = K.aa[13][11] != 0.0 ? fma(K.aa[13][11], ga[m], s.row[13][m]) : s.row[13][m];
+    q1[m] = fma(hh, a, fma(K.rs[SF - 1], hp[m], q[m]));
+    p1[m] = fma(h, s.row[SF][m], p[m]);
+    ep[m] = h * s.row[SF + 1][m];
+    eq[m] = fma(hh, s.row[SF + 2][m], K.se * hp[m]);
+    finite = finite && isfinite(q1[m]) && isfinite(p1[m]);
+  }
+  return finite;
+}
+
 // Wave 2: everything but the field.
 template <bool PID, class E, bool DENSE, bool TRACK>
 __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S,
                              int lane) {
   using M = Dopri8;
   constexpr int SF = M::SF;
-  constexpr auto& K = M::kf;
   const long long slot = (long long)blockIdx.x * kTeamOrbits + lane;
   // the first tickets of a cost-ordered queue: no second ticket for them in a
   // grid large enough for the rest to drain the queue
@@ -358,28 +502,8 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
       S.si[lane] = si;
     }
   };
-  // what the field and track waves need at the start of a step
-  auto publish = [&]() {
-    const double h = tnext - tau, hh = h * h;
-    S.hh[lane] = hh;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      const double hp = h * p[m];
-      S.x1[0][m][lane] = fma(M::kf.rs[1], hp, q[m]);
-      S.x1[1][m][lane] = fma(M::kf.rs[2], hp, q[m]);
-    }
-    if constexpr (TRACK) {
-      S.when[0][lane] = tau;
-      S.when[1][lane] = h;
-      S.when[2][lane] = tnext;
-      S.when[3][lane] = dir;
-    }
-  };
+  auto publish = [&]() { team_publish(S, lane, tau, tnext, dir, q, p); };
   int b = 0;  // the step's buffer of stage accelerations
-  auto load = [&](int l, double (&g)[3]) {
-#pragma unroll
-    for (int m = 0; m < 3; ++m) g[m] = S.g[b][l][m][lane];
-  };
 
   S.from_end[lane] = 0;
 #pragma unroll
@@ -394,91 +518,9 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
   if (!__any(orb >= 0)) return;
 
   for (;; b ^= TRACK ? 0 : 1) {
-    const double h = tnext - tau, hh = h * h;
-    const double hp[3] = {h * p[0], h * p[1], h * p[2]};
-    TeamSums s;
-#pragma unroll
-    for (int i = 0; i < kTeamSums; ++i) s.row[i][0] = s.row[i][1] = s.row[i][2] = 0.0;
-    // the next level's rows, for its two stages
-    auto hand_over = [&](auto level) {
-      constexpr int lv = decltype(level)::value;
-#pragma unroll
-      for (int w = 0; w < 2; ++w) {
-        constexpr int i0 = 2 * lv - 1;
-        if (i0 + w < SF) {
-#pragma unroll
-          for (int m = 0; m < 3; ++m) {
-            S.x[lv & 1][w][m][lane] = fma(M::kf.rs[i0 + w < SF ? i0 + w : 0], hp[m], q[m]);
-            S.x[lv & 1][w][m + 3][lane] = s.row[i0 + w < SF ? i0 + w : 0][m];
-          }
-        }
-      }
-    };
-    auto add_two = [&](auto first, const double (&g1)[3], const double (&g2)[3]) {
-      constexpr int L = decltype(first)::value;
-      ConstDouble* w = table_here(TeamWeights::t.w + TeamWeights::t.first[L]);
-      s.add<L, L, PID>(w, g1);
-      s.add<L + 1, L, PID>(w, g2);
-    };
-    double ga[3], gb[3];
-    // level 1: the start acceleration
-    if (TRACK) __syncthreads();
-    team_start(S, b, lane, ga);
-#pragma unroll
-    for (int m = 0; m < 3; ++m) S.start[m][lane] = S.g[b][0][m][lane] = ga[m];
-    s.add<0, 0, PID>(table_here(TeamWeights::t.w), ga);
-    hand_over(std::integral_constant<int, 2>{});
-    __syncthreads();
-    // levels 2 .. 6: the stages of the level before
-    if constexpr (!TRACK) {
-      S.begin[0][lane] = tau;
-      S.begin[1][lane] = h;
-#pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        S.begin[2 + m][lane] = q[m];
-        S.begin[5 + m][lane] = p[m];
-      }
-    }
-    load(1, ga);
-    load(2, gb);
-    add_two(std::integral_constant<int, 1>{}, ga, gb);
-    hand_over(std::integral_constant<int, 3>{});
-    __syncthreads();
-    load(3, ga);
-    load(4, gb);
-    add_two(std::integral_constant<int, 3>{}, ga, gb);
-    hand_over(std::integral_constant<int, 4>{});
-    __syncthreads();
-    load(5, ga);
-    load(6, gb);
-    add_two(std::integral_constant<int, 5>{}, ga, gb);
-    hand_over(std::integral_constant<int, 5>{});
-    __syncthreads();
-    load(7, ga);
-    load(8, gb);
-    add_two(std::integral_constant<int, 7>{}, ga, gb);
-    hand_over(std::integral_constant<int, 6>{});
-    __syncthreads();
-    load(9, ga);
-    load(10, gb);
-    add_two(std::integral_constant<int, 9>{}, ga, gb);
-    hand_over(std::integral_constant<int, 7>{});
-    __syncthreads();
-    // level 7: the step's end, beside the end stage
-    load(11, ga);
-    load(12, gb);
-    add_two(std::integral_constant<int, 11>{}, ga, gb);
+    const double h = tnext - tau;
     double q1[3], p1[3], eq[3], ep[3];
-    bool finite = true;
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      const double a = K.aa[13][11] != 0.0 ? fma(K.aa[13][11], ga[m], s.row[13][m]) : s.row[13][m];
-      q1[m] = fma(hh, a, fma(K.rs[SF - 1], hp[m], q[m]));
-      p1[m] = fma(h, s.row[SF][m], p[m]);
-      ep[m] = h * s.row[SF + 1][m];
-      eq[m] = fma(hh, s.row[SF + 2][m], K.se * hp[m]);
-      finite = finite && isfinite(q1[m]) && isfinite(p1[m]);
-    }
+    const bool finite = team_rows<PID, TRACK>(S, b, lane, tau, h, q, p, q1, p1, eq, ep);
     const double tau_s = tau, tend = tnext;
     const double qs[3] = {q[0], q[1], q[2]}, ps[3] = {p[0], p[1], p[2]};
     bool keep = false, done = false;
@@ -511,15 +553,7 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
     }
     S.from_end[lane] = keep ? 1 : 0;
     if constexpr (!TRACK) {
-      S.kept[lane] = keep ? 1 : 0;
-      if constexpr (DENSE) S.kept[lane] = keep ? (int)(nacc <= A.rec_cap ? nacc : A.rec_cap + 1) : 0;
-      S.done[lane] = done ? 1 : 0;
-      S.end[0][lane] = tend;
-#pragma unroll
-      for (int m = 0; m < 3; ++m) {
-        S.end[1 + m][lane] = q1[m];
-        S.end[4 + m][lane] = p1[m];
-      }
+      team_outcome(S, lane, keep, DENSE ? record_slot(nacc, A.rec_cap) : 1, done, tend, q1, p1);
     }
     const bool saves = TRACK && keep && si < A.T && !(tsave > tend);
     const bool serve = __any(done || saves);
@@ -532,7 +566,7 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
     if (saves) {
       double g[SF][3];
 #pragma unroll
-      for (int l = 0; l < SF; ++l) load(l, g[l]);
+      for (int l = 0; l < SF; ++l) team_stage_acc(S, b, l, lane, g[l]);
       while (si < A.T && !(tsave > tend)) {
         if (tsave == tend) {
           write_save(A, orb, si, dir, q1, p1);
@@ -562,8 +596,8 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
 // A lane's first save in the step is summed two stages a level; further ones
 // follow in the last level.  When some lane ends, all saves of the step come
 // before the team goes on.
-template <bool DENSE>
-__device__ void team_saves(const IArgs& A, TeamShared<false>& S, int lane) {
+template <bool DENSE, class Args>
+__device__ void team_saves(const Args& A, TeamShared<false>& S, int lane) {
   using M = Dopri8;
   constexpr int SF = M::SF;
   __syncthreads();
@@ -578,8 +612,7 @@ __device__ void team_saves(const IArgs& A, TeamShared<false>& S, int lane) {
     orb = S.orb[lane];
     si = S.si[lane];
     if (orb >= 0) {
-      t0v = A.t0[A.t_stride ? orb : 0];
-      t1v = A.t1[A.t_stride ? orb : 0];
+      orbit_span(A, orb, t0v, t1v);
       dir = (t0v < t1v) ? 1.0 : -1.0;
       next_save();
     }
@@ -598,10 +631,7 @@ __device__ void team_saves(const IArgs& A, TeamShared<false>& S, int lane) {
     }
   };
   auto due = [&]() { return kept != 0 && si < A.T && !(tsave > tend); };
-  auto load = [&](int b, int l, double (&g)[3]) {
-#pragma unroll
-    for (int m = 0; m < 3; ++m) g[m] = S.g[b][l][m][lane];
-  };
+  auto load = [&](int b, int l, double (&g)[3]) { team_stage_acc(S, b, l, lane, g); };
   auto write = [&](const double (&qo)[3], const double (&po)[3]) {
     if (tsave == tend)
       write_save(A, orb, si, dir, q1, p1);
