@@ -31,6 +31,7 @@ namespace gx {
 namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
 
@@ -207,18 +208,23 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
 }
 
 // The whole inference pass of an MLP of hidden width 256 in one kernel: a
-// block takes 64 points and keeps their activations in LDS (two 64 x 256
-// BF16 buffers, used in turn), so that activations never go to HBM; every
-// hidden-to-hidden layer runs on the matrix cores with the same operand
-// layout as k_gemm, the layer's BF16 weights read from L2 (each layer's
-// 128 KB is shared by every block).  Each wave owns 64 output columns of a
-// layer: 4 x 4 MFMA tiles.  The input layer (8 padded inputs) is a short
-// dot product in FP32 over the block's inputs staged in LDS; the output
-// layer (at most 16 columns, zero-padded) is one MFMA tile column per wave.
-// Rounding as the layer-by-layer path: FP32 accumulation, bias + SiLU in
-// FP32, BF16 activations.
+// block takes 128 points and keeps their activations in LDS, so that they
+// never go to HBM; every hidden-to-hidden layer runs on the matrix cores, the
+// layer's BF16 weights read from L2.  Each wave owns 64 output columns of a
+// layer: 8 x 4 MFMA tiles, weights as the first operand, so that a lane holds four neighbouring columns of a point and packs
+// its activations into one 8-byte LDS write.  A layer's results wait in
+// registers (as BF16) until all waves have read its inputs, so one buffer of
+// 68 KB serves and two blocks share a CU: one's matrix instructions run beside
+// the other's exponentials.  The input layer (8 padded inputs) is a short dot
+// product in FP32 over the block's inputs staged in LDS; the output layer (at
+// most 16 columns, zero-padded) is one MFMA tile column per wave.  Rounding as
+// the layer-by-layer path: FP32 accumulation, bias + SiLU in FP32, BF16
+// activations.  262,144 points (103 GFLOP): with 64 points a block 242 us,
+// bound by the weights' way from L2 (1.6 GB); with 128 and the next slab's
+// weights on their way 168 us (the products alone take 92 at the rate of a
+// large product, the exponentials and reciprocals some 90).
 constexpr int FH = 256;      // hidden width
-constexpr int FM = 64;       // points per block
+constexpr int FM = 128;      // points per block
 constexpr int FA = FM / 16;  // MFMA row tiles per block
 constexpr int FLD = FH + 8;  // padded LDS row (bf16 elements)
 constexpr int kMaxFusedLayers = 8;
@@ -235,8 +241,8 @@ struct FusedArgs {
   int ldy;
 };
 
-__global__ void __launch_bounds__(256) k_mlp_fused(FusedArgs f) {
-  __shared__ __bf16 act[2][FM][FLD];
+__global__ void __launch_bounds__(256, 2) k_mlp_fused(FusedArgs f) {
+  __shared__ __bf16 act[FM][FLD];
   __shared__ float xin[FM][8];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -264,49 +270,59 @@ __global__ void __launch_bounds__(256) k_mlp_fused(FusedArgs f) {
       float z = 0.0f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) z = fmaf(xin[r][k], w[k], z);
-      act[0][r][c] = (__bf16)silu(z + bias);
+      act[r][c] = (__bf16)silu(z + bias);
     }
   }
-  int cur = 0;
   // ---- hidden-to-hidden layers on the matrix cores
   for (int l = 1; l < f.depth; ++l) {
     __syncthreads();
     const __bf16* W = f.W[l];
+    const float* bias = f.b[l];
     f32x4 acc[FA][4];
 #pragma unroll
     for (int a = 0; a < FA; ++a)
 #pragma unroll
       for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __bf16* wl = W + (wave * 64 + (lane & 15)) * FH + (lane >> 4) * 8;
+    bf16x8 bw[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) bw[b] = *reinterpret_cast<const bf16x8*>(wl + b * 16 * FH);
 #pragma unroll 2
     for (int k0 = 0; k0 < FH; k0 += 32) {
-      const int kk = k0 + (lane >> 4) * 8;
-      bf16x8 af[FA], bw[4];
+      // the next slab's weights on their way during this one's products (the
+      // last slab loads its own again)
+      const int kn = k0 + 32 < FH ? k0 + 32 : k0;
+      bf16x8 next[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int n = wave * 64 + b * 16 + (lane & 15);
-        bw[b] = *reinterpret_cast<const bf16x8*>(W + n * FH + kk);
-      }
+      for (int b = 0; b < 4; ++b)
+        next[b] = *reinterpret_cast<const bf16x8*>(wl + b * 16 * FH + kn);
 #pragma unroll
-      for (int a = 0; a < FA; ++a)
-        af[a] = *reinterpret_cast<const bf16x8*>(&act[cur][a * 16 + (lane & 15)][kk]);
-#pragma unroll
-      for (int a = 0; a < FA; ++a)
+      for (int a = 0; a < FA; ++a) {
+        const bf16x8 af = *reinterpret_cast<const bf16x8*>(
+            &act[a * 16 + (lane & 15)][k0 + (lane >> 4) * 8]);
 #pragma unroll
         for (int b = 0; b < 4; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bw[b], acc[a][b], 0, 0, 0);
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[b], af, acc[a][b], 0, 0, 0);
+      }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) bw[b] = next[b];
     }
-    const float* bias = f.b[l];
+    bf16x4 out[FA][4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      const int n = wave * 64 + b * 16 + (lane & 15);
-      const float bn = bias[n];
+      const float* bn = bias + wave * 64 + b * 16 + (lane >> 4) * 4;
 #pragma unroll
       for (int a = 0; a < FA; ++a)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          act[cur ^ 1][a * 16 + (lane >> 4) * 4 + j][n] = (__bf16)silu(acc[a][b][j] + bn);
+        for (int j = 0; j < 4; ++j) out[a][b][j] = (__bf16)silu(acc[a][b][j] + bn[j]);
     }
-    cur ^= 1;
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < FA; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        *reinterpret_cast<bf16x4*>(
+            &act[a * 16 + (lane & 15)][wave * 64 + b * 16 + (lane >> 4) * 4]) = out[a][b];
   }
   __syncthreads();
   // ---- output layer on the matrix cores: wave w takes the 16-point row
@@ -332,7 +348,7 @@ __global__ void __launch_bounds__(256) k_mlp_fused(FusedArgs f) {
 #pragma unroll
       for (int s = 0; s < FH / 32; ++s) {
         const int kk = s * 32 + (lane >> 4) * 8;
-        const bf16x8 af = *reinterpret_cast<const bf16x8*>(&act[cur][a * 16 + n][kk]);
+        const bf16x8 af = *reinterpret_cast<const bf16x8*>(&act[a * 16 + n][kk]);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bw[s], acc, 0, 0, 0);
       }
       if (n < f.nout) {
