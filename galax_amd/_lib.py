@@ -88,6 +88,9 @@ SIGNATURES = {
     ),
     "gx_mlp_colsum": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "gx_mlp_adam": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _i64, _vp]),
+    "gx_mlp_adam_many": (
+        ctypes.c_int, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _f32, _f32, _f32, _i64, _vp],
+    ),
     "gx_mlp_huber": (ctypes.c_int, [_vp, _i64, _vp, _i64, _f32, _f32, _vp, _i64, _vp, _vp]),
     "gx_sur_inputs": (ctypes.c_int, [_vp, _vp, _i32, _f64, _i64, _f64, _f64, _vp, _i64, _vp]),
     "gx_sur_targets": (ctypes.c_int, [_vp, _i32, _i64, _vp, _vp, _f64, _f64, _vp, _vp]),

@@ -33,6 +33,7 @@ namespace {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
 typedef __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned u32x4;
 
 // x, or zero where keep is false, by a bit mask: loads feeding it stay
@@ -205,6 +206,289 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
           }
         }
       }
+}
+
+// Fragments of an operand whose memory holds columns side by side (rows along
+// k): a fragment wants eight k of one column, so a lane reads four columns (8
+// bytes) of its eight rows and repacks them in registers into four fragments.
+// Which columns make a tile is free: tile t holds columns 4 c + t of 64.
+// Columns beyond C read others' values into results that nobody stores; rows
+// from kend on count as zero (TAIL).
+template <bool TAIL>
+__device__ __forceinline__ void load_cols(u32x2 (&v)[8], const __bf16* X, long long sk,
+                                          long long k, long long kend) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    v[j] = *reinterpret_cast<const u32x2*>(X + (!TAIL || k + j < kend ? k + j : kend - 1) * sk);
+  if (TAIL) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const unsigned mask = k + j < kend ? ~0u : 0u;
+      v[j] = u32x2{v[j][0] & mask, v[j][1] & mask};
+    }
+  }
+}
+// Fragment t (of four): column t of the eight rows.
+__device__ __forceinline__ bf16x8 fragment(const u32x2 (&v)[8], int t) {
+  u32x4 f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    f[j] = __builtin_amdgcn_perm(v[2 * j + 1][t >> 1], v[2 * j][t >> 1],
+                                 t & 1 ? 0x07060302u : 0x05040100u);
+  return __builtin_bit_cast(bf16x8, f);
+}
+
+// The large products whose A is read along k (the layers' forward passes and
+// the activations' gradients).  Such a product moves 2 (A, H) + 4 (C or Zin)
+// bytes an element and is bound by memory: 65,536 x 256 x 256 is 134 MB, 26 us
+// at the rate of a copy.  A block takes 128 x 128 of C, a wave 64 x 64 as 4 x
+// 4 MFMA tiles.  Fragments come straight from memory, a slab ahead of the
+// products: A's from HBM, the weights' from L2, along k (BK_ROWS) or as columns.
+// The operands are swapped (D = B^T A^T), so that a lane holds four
+// neighbouring columns of a row (or, of a columns' B, the four tiles do), and
+// the results pass through LDS to leave in whole rows: 16-byte stores of C,
+// 8-byte stores of H, 16-byte loads of Zin.  64 x 64 tiles read A four times
+// and stored single elements.  Each
+// element's sum runs over k in the order of k_gemm, so the bits are the same.
+constexpr int RM = 128, RN = 128;
+
+constexpr int RLD = 64 + 4;  // padded LDS row of a wave's results
+
+// LDS that only one wave uses: its writes are done before its later reads
+// (LDS works in order), the compiler keeps them so.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <bool BROWS>
+__global__ void __launch_bounds__(256, 2) k_gemm_rows(GemmArgs g, int ntiles) {
+  __shared__ float T[4][16][RLD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // Blocks go to the eight XCDs in turn: the n tiles of one m tile are eight
+  // blocks apart, so that A's rows are read by one XCD.
+  const unsigned group = blockIdx.x / (8 * ntiles), in = blockIdx.x % (8 * ntiles);
+  const long long m0 = ((long long)group * 8 + in % 8) * RM, n0 = (long long)(in / 8) * RN;
+  if (m0 >= g.M) return;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const int kl = (lane >> 4) * 8;
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // this lane's rows of A and of B, or B's four columns (in range: rows and
+  // columns beyond the end stand for the last)
+  const __bf16 *pa[4], *pb[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const long long m = m0 + wm + a * 16 + (lane & 15);
+    pa[a] = g.A + (m < g.M ? m : g.M - 1) * g.sam;
+    if (BROWS) {
+      const long long n = n0 + wn + a * 16 + (lane & 15);
+      pb[a] = g.B + (n < g.N ? n : g.N - 1) * g.sbn;
+    }
+  }
+  const long long nc = n0 + wn + (lane & 15) * 4;
+  const __bf16* cols = g.B + (nc < g.N ? nc : 0);
+  struct Slab {
+    u32x4 a[4], b[4];
+    u32x2 c[8];
+  };
+  // k from K on (K is a multiple of eight) counts as zero
+  auto load = [&](Slab& s, long long k0) {
+    const long long k = k0 + kl;
+    const bool keep = k < g.K;
+    const long long kk = keep ? k : 0;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      s.a[a] = *reinterpret_cast<const u32x4*>(pa[a] + kk);
+      if (BROWS) s.b[a] = *reinterpret_cast<const u32x4*>(pb[a] + kk);
+    }
+    if (!BROWS) load_cols<false>(s.c, cols, g.sbk, kk, 0);
+  };
+  auto products = [&](const Slab& s, long long k0) {
+    const unsigned mask = k0 + kl < g.K ? ~0u : 0u;
+    bf16x8 bf[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      bf[b] = BROWS ? __builtin_bit_cast(bf16x8, s.b[b] & mask)
+                    : __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, fragment(s.c, b)) & mask);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const bf16x8 af = __builtin_bit_cast(bf16x8, s.a[a] & mask);
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[b], af, acc[a][b], 0, 0, 0);
+    }
+  };
+  Slab s0, s1;
+  load(s0, 0);
+  for (long long k0 = 0; k0 < g.K; k0 += 2 * BK) {
+    load(s1, k0 + BK);
+    products(s0, k0);
+    load(s0, k0 + 2 * BK);
+    products(s1, k0 + BK);
+  }
+  const auto aligned = [](const void* q, int bytes) {
+    return (reinterpret_cast<uintptr_t>(q) & (bytes - 1)) == 0;
+  };
+  // sixteen rows at a time through the wave's own LDS, so that a row's 64
+  // columns are loaded and stored together
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    float(&t)[16][RLD] = T[wave];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      f32x4 c = acc[a][b];
+      if (!BROWS) c = f32x4{acc[a][0][b], acc[a][1][b], acc[a][2][b], acc[a][3][b]};
+      const int col = BROWS ? b * 16 + (lane >> 4) * 4 : (lane >> 4) * 16 + b * 4;
+      *reinterpret_cast<f32x4*>(&t[lane & 15][col]) = c;
+    }
+    wave_lds_fence();
+    f32x4 rows[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      rows[i] = *reinterpret_cast<const f32x4*>(&t[i * 4 + (lane >> 4)][(lane & 15) * 4]);
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const long long m = m0 + wm + a * 16 + i * 4 + (lane >> 4);
+      const long long n = n0 + wn + (lane & 15) * 4;
+      if (m >= g.M || n >= g.N) continue;
+      const int cols = g.N - n < 4 ? (int)(g.N - n) : 4;
+      float* C = g.C ? g.C + m * g.ldc + n : nullptr;
+      __bf16* H = g.H ? g.H + m * g.ldh + n : nullptr;
+      f32x4 c = rows[i];
+      bf16x4 h = {};
+      if (g.epi == EPI_DSILU) {
+        const float* Z = g.Zin + m * g.ldzin + n;
+        f32x4 z = {};
+        if (cols == 4 && aligned(Z, 16)) {
+          z = *reinterpret_cast<const f32x4*>(Z);
+        } else {
+          for (int j = 0; j < cols; ++j) z[j] = Z[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) h[j] = (__bf16)(c[j] * dsilu(z[j]));
+      } else if (g.epi != EPI_STORE) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          c[j] += g.bias[n + (j < cols ? j : 0)];
+          h[j] = (__bf16)silu(c[j]);
+        }
+      } else if (g.accumulate) {
+        for (int j = 0; j < cols; ++j) c[j] += C[j];
+      }
+      if (g.epi != EPI_DSILU && C) {
+        if (cols == 4 && aligned(C, 16)) {
+          *reinterpret_cast<f32x4*>(C) = c;
+        } else {
+          for (int j = 0; j < cols; ++j) C[j] = c[j];
+        }
+      }
+      if (g.epi == EPI_BIAS_SILU || g.epi == EPI_DSILU) {
+        if (cols == 4 && aligned(H, 8)) {
+          *reinterpret_cast<bf16x4*>(H) = h;
+        } else {
+          for (int j = 0; j < cols; ++j) H[j] = h[j];
+        }
+      }
+    }
+  }
+}
+
+// The weights' gradients C = sum_k A(m, k) B(k, n) with both operands' rows
+// along k (dZ^T H over the batch), fragments straight from memory as columns.
+// A block takes 128 x 128 of C over its share of k, four waves 64 x 64 each
+// and a second four every other slab; their sums meet in LDS and leave it in
+// whole rows.  65,536 x 256 x 256 is 67 MB, 13 us at the rate of a copy, and 17
+// MB of atomic sums: 78 -> 37 us.  (Through LDS, transposed by 2-byte writes,
+// a slab waited for its own loads.)
+constexpr int kColsLd = 128 + 4;
+
+__global__ void __launch_bounds__(512, 2) k_gemm_cols(GemmArgs g) {
+  __shared__ float T[128][kColsLd];
+  const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const long long mb = (long long)blockIdx.x * 128, nb = (long long)blockIdx.y * 128;
+  const long long mc = mb + wm + (lane & 15) * 4, nc = nb + wn + (lane & 15) * 4;
+  const __bf16* A = g.A + (mc < g.M ? mc : 0);
+  const __bf16* B = g.B + (nc < g.N ? nc : 0);
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const long long kper = ((g.K + g.ksplit - 1) / g.ksplit + BK - 1) / BK * BK;
+  const long long kbeg = (long long)blockIdx.z * kper;
+  const long long kend = kbeg + kper < g.K ? kbeg + kper : g.K;
+  if (kbeg >= kend) return;
+  const int kl = (lane >> 4) * 8;
+  auto products = [&](const u32x2 (&va)[8], const u32x2 (&vb)[8]) {
+    bf16x8 af[4], bf[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      af[t] = fragment(va, t);
+      bf[t] = fragment(vb, t);
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bf[b], acc[a][b], 0, 0, 0);
+  };
+  // whole slabs, two on their way (beyond the last the first is read again)
+  const long long whole = kbeg + (kend - kbeg) / BK * BK;
+  const long long first = kbeg + half * BK;
+  u32x2 va[2][8], vb[2][8];
+  auto load = [&](int s, long long k0) {
+    const long long k = (k0 < whole ? k0 : kbeg) + kl;
+    load_cols<false>(va[s], A, g.sak, k, 0);
+    load_cols<false>(vb[s], B, g.sbk, k, 0);
+  };
+  if (first < whole) {
+    load(0, first);
+    load(1, first + 2 * BK);
+    for (long long k0 = first; k0 < whole; k0 += 4 * BK) {
+      products(va[0], vb[0]);
+      load(0, k0 + 4 * BK);
+      if (k0 + 2 * BK < whole) products(va[1], vb[1]);
+      load(1, k0 + 6 * BK);
+    }
+  }
+  if (whole < kend && half == 0) {
+    load_cols<true>(va[0], A, g.sak, whole + kl, kend);
+    load_cols<true>(vb[0], B, g.sbk, whole + kl, kend);
+    products(va[0], vb[0]);
+  }
+  // tile (a, b), entry j: row 4 (4 (l / 16) + j) + a, column 4 (l % 16) + b
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (half == h) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f32x4* t = reinterpret_cast<f32x4*>(
+              &T[wm + 4 * ((lane >> 4) * 4 + j) + a][wn + (lane & 15) * 4]);
+          f32x4 v = f32x4{acc[a][0][j], acc[a][1][j], acc[a][2][j], acc[a][3][j]};
+          if (h == 1) v += *t;
+          *t = v;
+        }
+    }
+    __syncthreads();
+  }
+  const int c = threadIdx.x & 127;
+  if (nb + c >= g.N) return;
+  for (int r = threadIdx.x >> 7; r < 128 && mb + r < g.M; r += 4) {
+    float* C = g.C + (mb + r) * g.ldc + nb + c;
+    const float v = T[r][c];
+    if (g.ksplit > 1)
+      atomicAdd(C, v);
+    else
+      *C = g.accumulate ? *C + v : v;
+  }
 }
 
 // The whole inference pass of an MLP of hidden width 256 in one kernel: a
@@ -388,22 +672,89 @@ __global__ void k_colsum(const __bf16* __restrict__ dz, long long ld, long long 
   atomicAdd(out + n, (s0 + s1) + (s2 + s3));
 }
 
+// The same for rows of 16-byte alignment and whole groups of eight columns
+// (the hidden layers): a lane reads eight columns at a time, and a block's
+// partial sums meet in LDS before the atomics.  65,536 x 256: 22 -> 18 us (7
+// at the rate of a copy; the sums into one row of results are the rest).
+constexpr int kColsumGroups = 32;  // groups of eight columns a block covers
+__global__ void __launch_bounds__(256) k_colsum8(const __bf16* __restrict__ dz, long long ld,
+                                                 long long M, long long N,
+                                                 float* __restrict__ out) {
+  __shared__ float part[8][kColsumGroups][8 + 1];
+  const int c = threadIdx.x % kColsumGroups, r = threadIdx.x / kColsumGroups;
+  const long long n = ((long long)blockIdx.x * kColsumGroups + c) * 8;
+  const long long rows = (M + gridDim.y - 1) / gridDim.y;
+  const long long r0 = (long long)blockIdx.y * rows;
+  const long long r1 = r0 + rows < M ? r0 + rows : M;
+  float s[2][8] = {};
+  if (n < N) {
+    long long m = r0 + r;
+    for (; m + 8 < r1; m += 16) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(dz + m * ld + n);
+      const bf16x8 w = *reinterpret_cast<const bf16x8*>(dz + (m + 8) * ld + n);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        s[0][j] += (float)v[j];
+        s[1][j] += (float)w[j];
+      }
+    }
+    if (m < r1) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(dz + m * ld + n);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[0][j] += (float)v[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) part[r][c][j] = s[0][j] + s[1][j];
+  __syncthreads();
+  const int cc = threadIdx.x >> 3, j = threadIdx.x & 7;
+  const long long col = ((long long)blockIdx.x * kColsumGroups + cc) * 8 + j;
+  if (col >= N) return;
+  float t = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) t += part[k][cc][j];
+  atomicAdd(out + col, t);
+}
+
 // Adam on fp32 master parameters (bias-corrected, as Kingma & Ba 2015);
 // writes the bf16 copy the GEMMs read.
+struct AdamStep {
+  float lr, b1, b2, eps, c1, c2;
+  __device__ __forceinline__ void at(float* p, const float* g, float* m, float* v, __bf16* pb,
+                                     long long i) const {
+    const float gi = g[i];
+    const float mi = b1 * m[i] + (1.f - b1) * gi;
+    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float pi = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+    p[i] = pi;
+    if (pb) pb[i] = (__bf16)pi;
+  }
+};
+
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g,
                        float* __restrict__ m, float* __restrict__ v,
-                       __bf16* __restrict__ pb, long long n, float lr, float b1,
-                       float b2, float eps, float c1, float c2) {
+                       __bf16* __restrict__ pb, long long n, AdamStep s) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-  p[i] = pi;
-  if (pb) pb[i] = (__bf16)pi;
+  if (i < n) s.at(p, g, m, v, pb, i);
+}
+
+// Several tensors in one launch (grid y): ten launches of a network's weights
+// and biases took 45 us, one takes 5.
+constexpr int kAdamTensors = GX_ADAM_TENSORS;
+struct AdamTensors {
+  float* p[kAdamTensors];
+  const float* g[kAdamTensors];
+  float *m[kAdamTensors], *v[kAdamTensors];
+  __bf16* pb[kAdamTensors];
+  long long n[kAdamTensors];
+};
+__global__ void k_adam_many(AdamTensors a, AdamStep s) {
+  const int k = blockIdx.y;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < a.n[k];
+       i += (long long)gridDim.x * blockDim.x)
+    s.at(a.p[k], a.g[k], a.m[k], a.v[k], a.pb[k], i);
 }
 
 // Pseudo-Huber loss on the network's outputs: r = Y - T (first 3 columns),
@@ -588,6 +939,11 @@ long long blocks_for(long long n, int bs) { return (n + bs - 1) / bs; }
 
 bool grid_ok(long long n) { return blocks_for(n, 256) <= 0x7fffffffLL; }
 
+AdamStep adam_step(float lr, float b1, float b2, float eps, int64_t step) {
+  return {lr, b1, b2, eps, 1.0f / (1.0f - powf(b1, (float)step)),
+          1.0f / (1.0f - powf(b2, (float)step))};
+}
+
 }  // namespace
 }  // namespace gx
 
@@ -628,6 +984,39 @@ int gx_mlp_gemm(const void* A, int64_t sam, int64_t sak, const void* B,
   g.ldh = ldh;
   g.Zin = Zin;
   g.ldzin = ldzin;
+  // Both operands' rows along k: the kernel that reads them so, from a wave's
+  // tile on (a network's first layer, N = 8, takes 27 us with k_gemm at K =
+  // 65,536 and 31 with this) and from K where its blocks have a few slabs each
+  // (256 x 256 x 2,048: 10.7 / 11.3 us; 4,096: 13.2 / 11.4; 65,536: 78 / 37).
+  if (epi == EPI_STORE && sam == 1 && sbn == 1 && M >= 64 && N >= 64 && M % 4 == 0 &&
+      N % 4 == 0 && sak % 4 == 0 && sbk % 4 == 0 && K >= 3072 &&
+      (reinterpret_cast<uintptr_t>(A) & 7) == 0 && (reinterpret_cast<uintptr_t>(B) & 7) == 0 &&
+      (M + 127) / 128 <= 0x7fffffffLL && (N + 127) / 128 <= 65535) {
+    hipLaunchKernelGGL(k_gemm_cols,
+                       dim3((unsigned)((M + 127) / 128), (unsigned)((N + 127) / 128),
+                            (unsigned)ksplit),
+                       dim3(512), 0, (hipStream_t)stream, g);
+    return check(hipGetLastError());
+  }
+  // A along k: 128 x 128 tiles where they fill the device several times, which
+  // hides a block's start and end.  x 256 x 256 with SiLU / its derivative, us,
+  // k_gemm then this: 16,384 rows 16 21 / 23 27; 24,576 26 29 / 34 29; 32,768
+  // 29 30 / 38 30; 49,152 42 39 / 53 34; 65,536 57 51 / 71 41.
+  const long long rt = (M + RM - 1) / RM, ct = (N + RN - 1) / RN;
+  const auto aligned = [](const void* q, int bytes) {
+    return (reinterpret_cast<uintptr_t>(q) & (bytes - 1)) == 0;
+  };
+  const bool brows = sbk == 1 && sbn % 8 == 0 && aligned(B, 16);
+  const bool bcols = sbn == 1 && sbk % 4 == 0 && aligned(B, 8) && N % 4 == 0;
+  if (sak == 1 && sam % 8 == 0 && aligned(A, 16) && K % 8 == 0 && K > 0 && ksplit == 1 &&
+      N >= 64 && (brows || bcols) && rt * ct >= (epi == EPI_DSILU ? 384 : 640) &&
+      rt * ct < 0x7fffff00LL) {
+    const long long groups = (rt + 7) / 8;
+    const auto kern = brows ? k_gemm_rows<true> : k_gemm_rows<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(groups * 8 * ct)), dim3(256), 0, (hipStream_t)stream,
+                       g, (int)ct);
+    return check(hipGetLastError());
+  }
   const long long mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
   if (mt > 0x7fffffffLL || nt > 65535) return GX_EINVAL;
   dim3 grid((unsigned)mt, (unsigned)nt, (unsigned)ksplit);
@@ -673,6 +1062,12 @@ int gx_mlp_colsum(const void* dz, int64_t ld, int64_t M, int64_t N, float* out,
   if (M == 0 || N == 0) return GX_OK;
   long long ychunks = (M + kColsumRows - 1) / kColsumRows;
   if (ychunks > 65535) ychunks = 65535;  // grid y limit; chunks then grow
+  if (N % 8 == 0 && ld % 8 == 0 && (reinterpret_cast<uintptr_t>(dz) & 15) == 0) {
+    hipLaunchKernelGGL(k_colsum8, dim3((unsigned)blocks_for(N, 8 * kColsumGroups), (unsigned)ychunks),
+                       dim3(256), 0, (hipStream_t)stream, static_cast<const __bf16*>(dz),
+                       (long long)ld, (long long)M, (long long)N, out);
+    return check(hipGetLastError());
+  }
   dim3 grid((unsigned)blocks_for(N, 256), (unsigned)ychunks);
   hipLaunchKernelGGL(k_colsum, grid, dim3(256), 0, (hipStream_t)stream,
                      static_cast<const __bf16*>(dz), (long long)ld, (long long)M,
@@ -686,11 +1081,34 @@ int gx_mlp_adam(float* p, const float* g, float* m, float* v, void* pb,
   if (!p || !g || !m || !v || n < 0 || step < 1) return GX_EINVAL;
   if (n == 0) return GX_OK;
   if (!grid_ok(n)) return GX_EINVAL;
-  const float c1 = 1.0f / (1.0f - powf(b1, (float)step));
-  const float c2 = 1.0f / (1.0f - powf(b2, (float)step));
   hipLaunchKernelGGL(k_adam, dim3((unsigned)blocks_for(n, 256)), dim3(256), 0,
                      (hipStream_t)stream, p, g, m, v, static_cast<__bf16*>(pb),
-                     (long long)n, lr, b1, b2, eps, c1, c2);
+                     (long long)n, adam_step(lr, b1, b2, eps, step));
+  return check(hipGetLastError());
+}
+
+int gx_mlp_adam_many(int32_t count, float* const* p, const float* const* g, float* const* m,
+                     float* const* v, void* const* pb, const int64_t* n, float lr, float b1,
+                     float b2, float eps, int64_t step, void* stream) {
+  if (count < 0 || count > kAdamTensors || step < 1) return GX_EINVAL;
+  if (count == 0) return GX_OK;
+  if (!p || !g || !m || !v || !pb || !n) return GX_EINVAL;
+  AdamTensors a{};
+  long long most = 0;
+  for (int k = 0; k < count; ++k) {
+    if (n[k] < 0 || (n[k] > 0 && (!p[k] || !g[k] || !m[k] || !v[k]))) return GX_EINVAL;
+    a.p[k] = p[k];
+    a.g[k] = g[k];
+    a.m[k] = m[k];
+    a.v[k] = v[k];
+    a.pb[k] = static_cast<__bf16*>(pb[k]);
+    a.n[k] = n[k];
+    if (n[k] > most) most = n[k];
+  }
+  if (most == 0) return GX_OK;
+  const long long blocks = blocks_for(most, 256) < 4096 ? blocks_for(most, 256) : 4096;
+  hipLaunchKernelGGL(k_adam_many, dim3((unsigned)blocks, (unsigned)count), dim3(256), 0,
+                     (hipStream_t)stream, a, adam_step(lr, b1, b2, eps, step));
   return check(hipGetLastError());
 }
 

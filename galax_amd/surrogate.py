@@ -157,8 +157,7 @@ class MLP:
         dY[n][K_IN] (bf16, first 3 columns used) after forward(train=True)."""
         torch = _lib.torch()
         h, L = self.hidden, self.depth
-        for g in self.g:
-            g.zero_()
+        torch._foreach_zero_(self.g)  # one launch
         gW, gb = self.g[: L + 1], self.g[L + 1 :]
         # output layer
         Hl = self._bufs[("H", L - 1)]
@@ -179,11 +178,15 @@ class MLP:
 
     def adam(self, lr, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1
-        nW = len(self.W)
-        for i, (p, g, m, v) in enumerate(zip(self.params, self.g, self.m, self.v)):
-            pb = self.Wb[i] if i < nW else None
-            rc = _L().gx_mlp_adam(_p(p), _p(g), _p(m), _p(v), _p(pb), p.numel(), lr, b1, b2, eps, self.step, _s())
-            _lib.check(rc, "gx_mlp_adam")
+        pb = [_p(w) for w in self.Wb] + [None] * len(self.b)
+        rows = [[_p(x) for x in xs] for xs in (self.params, self.g, self.m, self.v)] + [pb]
+        sizes = [p.numel() for p in self.params]
+        for i in range(0, len(sizes), _abi.GX_ADAM_TENSORS):
+            part = sizes[i:i + _abi.GX_ADAM_TENSORS]
+            k = len(part)
+            tabs = [(ctypes.c_void_p * k)(*r[i:i + k]) for r in rows]
+            rc = _L().gx_mlp_adam_many(k, *tabs, (ctypes.c_int64 * k)(*part), lr, b1, b2, eps, self.step, _s())
+            _lib.check(rc, "gx_mlp_adam_many")
 
     def train_step(self, X, T, n, lr, delta=1.0, loss=None):
         """One Adam step on the pseudo-Huber loss of MLP(X) against T[n][3];

@@ -462,6 +462,13 @@ int gx_mlp_colsum(const void* dz, int64_t ld, int64_t M, int64_t N, float* out,
 int gx_mlp_adam(float* p, const float* g, float* m, float* v, void* pb,
                 int64_t n, float lr, float b1, float b2, float eps, int64_t step,
                 void* stream);
+/* The same for up to GX_ADAM_TENSORS tensors in one launch (arrays of `count`
+ * host-side pointers and sizes; pb[k] may be null). */
+#define GX_ADAM_TENSORS 20
+int gx_mlp_adam_many(int32_t count, float* const* p, const float* const* g,
+                     float* const* m, float* const* v, void* const* pb,
+                     const int64_t* n, float lr, float b1, float b2, float eps,
+                     int64_t step, void* stream);
 /* Pseudo-Huber loss of Y[:, 0:3] (row stride ldy) against T[B][3]:
  * *loss += sum delta^2 (sqrt(1 + (r/delta)^2) - 1) (loss must hold the
  * start), dY[:, 0:3] = bf16(scale * r / sqrt(1 + (r/delta)^2)), other
