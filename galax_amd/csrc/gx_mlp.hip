@@ -504,12 +504,10 @@ __global__ void __launch_bounds__(512, 2) k_gemm_cols(GemmArgs g) {
 // most 16 columns, zero-padded) is one MFMA tile column per wave.  Rounding as
 // the layer-by-layer path: FP32 accumulation, bias + SiLU in FP32, BF16
 // activations.  262,144 points (103 GFLOP): with 64 points a block 242 us,
-// bound by the weights' way from L2 (1.6 GB); with 128 and the next slab's
+// bound by the weights' way from L2 (1.6 GB); with 128 (FA = 8) and the next slab's
 // weights on their way 168 us (the products alone take 92 at the rate of a
 // large product, the exponentials and reciprocals some 90).
 constexpr int FH = 256;      // hidden width
-constexpr int FM = 128;      // points per block
-constexpr int FA = FM / 16;  // MFMA row tiles per block
 constexpr int FLD = FH + 8;  // padded LDS row (bf16 elements)
 constexpr int kMaxFusedLayers = 8;
 
@@ -525,7 +523,9 @@ struct FusedArgs {
   int ldy;
 };
 
+template <int FA>  // MFMA row tiles per block, of 16 points each
 __global__ void __launch_bounds__(256, 2) k_mlp_fused(FusedArgs f) {
+  constexpr int FM = 16 * FA;
   __shared__ __bf16 act[FM][FLD];
   __shared__ float xin[FM][8];
   const int tid = threadIdx.x;
@@ -1049,9 +1049,15 @@ int gx_mlp_forward_fused(const void* X, int32_t ldx, int32_t nin, int64_t n,
     f.W[l] = static_cast<const __bf16*>(W[l]);
     f.b[l] = b[l];
   }
-  const long long blocks = (n + FM - 1) / FM;
+  // 64 points a block while each still has a CU of its own, where a block's
+  // latency is all (us with 64 / 128 points: 100 points 23 / 32, 16,384 25 /
+  // 33; 24,576 34 / 33, 65,536 59 / 43, 262,144 216 / 168)
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return GX_ELAUNCH;
+  const bool small = n <= 64LL * num_cus(dev);
+  const long long blocks = (n + (small ? 63 : 127)) / (small ? 64 : 128);
   if (blocks > 0x7fffffffLL) return GX_EINVAL;
-  hipLaunchKernelGGL(k_mlp_fused, dim3((unsigned)blocks), dim3(256), 0,
+  hipLaunchKernelGGL(small ? k_mlp_fused<4> : k_mlp_fused<8>, dim3((unsigned)blocks), dim3(256), 0,
                      (hipStream_t)stream, f);
   return check(hipGetLastError());
 }

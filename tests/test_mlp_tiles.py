@@ -81,7 +81,7 @@ def test_column_sums(M, N):
     assert bool(((out - X.float().sum(0)).abs() <= 2 * M * EPS32 * X.float().abs().sum(0)).all())
 
 
-@pytest.mark.parametrize("n", [1, 127, 128, 129, 300])
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 300, 16385, 16513])
 @pytest.mark.parametrize("depth", [1, 2, 4])
 def test_fused_inference_follows_the_layers(n, depth):
 
