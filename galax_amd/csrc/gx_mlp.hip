@@ -674,13 +674,16 @@ __global__ void k_colsum(const __bf16* __restrict__ dz, long long ld, long long 
 
 // The same for rows of 16-byte alignment and whole groups of eight columns
 // (the hidden layers): a lane reads eight columns at a time, and a block's
-// partial sums meet in LDS before the atomics.  65,536 x 256: 22 -> 18 us (7
-// at the rate of a copy; the sums into one row of results are the rest).
-constexpr int kColsumGroups = 32;  // groups of eight columns a block covers
-__global__ void __launch_bounds__(256) k_colsum8(const __bf16* __restrict__ dz, long long ld,
+// partial sums meet in LDS before the atomics, which are what bounds it: 512
+// blocks of 128 rows took 18 us for 65,536 x 256, 128 blocks of 512 rows 9 (7
+// at the rate of a copy; a lane a column: 22).
+constexpr int kColsumGroups = 32;    // groups of eight columns a block covers
+constexpr int kColsumLanes = 32;     // rows it reads side by side
+constexpr int kColsum8Rows = 512;    // rows of a block
+__global__ void __launch_bounds__(kColsumGroups * kColsumLanes) k_colsum8(const __bf16* __restrict__ dz, long long ld,
                                                  long long M, long long N,
                                                  float* __restrict__ out) {
-  __shared__ float part[8][kColsumGroups][8 + 1];
+  __shared__ float part[kColsumLanes][kColsumGroups][8 + 1];
   const int c = threadIdx.x % kColsumGroups, r = threadIdx.x / kColsumGroups;
   const long long n = ((long long)blockIdx.x * kColsumGroups + c) * 8;
   const long long rows = (M + gridDim.y - 1) / gridDim.y;
@@ -689,9 +692,9 @@ __global__ void __launch_bounds__(256) k_colsum8(const __bf16* __restrict__ dz, 
   float s[2][8] = {};
   if (n < N) {
     long long m = r0 + r;
-    for (; m + 8 < r1; m += 16) {
+    for (; m + kColsumLanes < r1; m += 2 * kColsumLanes) {
       const bf16x8 v = *reinterpret_cast<const bf16x8*>(dz + m * ld + n);
-      const bf16x8 w = *reinterpret_cast<const bf16x8*>(dz + (m + 8) * ld + n);
+      const bf16x8 w = *reinterpret_cast<const bf16x8*>(dz + (m + kColsumLanes) * ld + n);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         s[0][j] += (float)v[j];
@@ -707,12 +710,13 @@ __global__ void __launch_bounds__(256) k_colsum8(const __bf16* __restrict__ dz, 
 #pragma unroll
   for (int j = 0; j < 8; ++j) part[r][c][j] = s[0][j] + s[1][j];
   __syncthreads();
+  if (threadIdx.x >= 8 * kColsumGroups) return;
   const int cc = threadIdx.x >> 3, j = threadIdx.x & 7;
   const long long col = ((long long)blockIdx.x * kColsumGroups + cc) * 8 + j;
   if (col >= N) return;
   float t = 0.f;
 #pragma unroll
-  for (int k = 0; k < 8; ++k) t += part[k][cc][j];
+  for (int k = 0; k < kColsumLanes; ++k) t += part[k][cc][j];
   atomicAdd(out + col, t);
 }
 
@@ -1069,8 +1073,10 @@ int gx_mlp_colsum(const void* dz, int64_t ld, int64_t M, int64_t N, float* out,
   long long ychunks = (M + kColsumRows - 1) / kColsumRows;
   if (ychunks > 65535) ychunks = 65535;  // grid y limit; chunks then grow
   if (N % 8 == 0 && ld % 8 == 0 && (reinterpret_cast<uintptr_t>(dz) & 15) == 0) {
+    ychunks = (M + kColsum8Rows - 1) / kColsum8Rows;
+    if (ychunks > 65535) ychunks = 65535;
     hipLaunchKernelGGL(k_colsum8, dim3((unsigned)blocks_for(N, 8 * kColsumGroups), (unsigned)ychunks),
-                       dim3(256), 0, (hipStream_t)stream, static_cast<const __bf16*>(dz),
+                       dim3(kColsumGroups * kColsumLanes), 0, (hipStream_t)stream, static_cast<const __bf16*>(dz),
                        (long long)ld, (long long)M, (long long)N, out);
     return check(hipGetLastError());
   }
