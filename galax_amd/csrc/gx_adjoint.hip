@@ -506,8 +506,10 @@ extern "C" {
 
 int64_t gx_adjoint_workspace_bytes(int64_t n, int64_t max_steps, int32_t K) {
   if (n < 0 || max_steps < 0 || K < 1) return 0;
-  return all_states(n, max_steps, K) ? 56 * n * step_limit(max_steps, K) + 256
-                                     : 56 * n * (max_steps / K + 2 + K) + 256;
+  if (all_states(n, max_steps, K)) return 56 * n * step_limit(max_steps, K) + 256;
+  // not less than any smaller batch or span takes, whose states may all be kept
+  const int64_t checkpointed = 56 * n * (max_steps / K + 2 + K);
+  return (checkpointed > kAllStatesBytes ? checkpointed : kAllStatesBytes) + 256;
 }
 
 int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,

@@ -369,7 +369,7 @@ int gx_integrate_shared(const gx_pot* pot, const gx_solver_cfg* cfg,
  * State is checkpointed every K steps, or at every step where that takes
  * at most 4 GiB; max_steps bounds the steps of any
  * orbit (it sizes the workspace, gx_adjoint_workspace_bytes(n, max_steps,
- * K) bytes, 256-byte aligned).  status[n] (optional) is GX_SUCCESS or
+ * K) bytes, 256-byte aligned, which also serve any smaller n or max_steps).  status[n] (optional) is GX_SUCCESS or
  * GX_MAX_STEPS_REACHED.  Replaces differentiating evaluate_orbit /
  * MockStreamGenerator.run with jax (dynamics/_src/orbit/solver.py:133,
  * tests/functional/test_mockstreamgenerator.py:24-116). */
