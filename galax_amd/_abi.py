@@ -66,6 +66,7 @@ GX_TS_LINSPACE = 2
 GX_TS_FINAL = 3
 
 GX_DENSE_RECORD = 50
+GX_ADJOINT_STATES_BYTES = 4 << 30  # states that gx_adjoint keeps at most for every step
 GX_ADAM_TENSORS = 20  # tensors of one gx_mlp_adam_many call
 
 GX_MAX_COMPONENTS = 256

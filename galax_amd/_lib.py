@@ -76,6 +76,11 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _i64, _vp, _vp, _vp, _i32, _i64, _i32, _vp, _vp, _vp],
     ),
+    "gx_adjoint_workspace_within": (_i64, [_i64, _i64, _i32, _i64]),
+    "gx_adjoint_within": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _i64, _vp, _vp, _vp, _i32, _i64, _i32, _vp, _vp, _i64, _vp],
+    ),
     # surrogate kernels
     "gx_mlp_gemm": (
         ctypes.c_int,

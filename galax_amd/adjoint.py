@@ -36,10 +36,14 @@ def steps_bound(t0, t1, dt0: float) -> int:
 
 
 def adjoint_orbits(pot, w0, t0, t1, cot, *, dt0: float, ts=None, method=None, K: int = 64,
-                   ntheta: int = 0, max_steps: int | None = None):
+                   ntheta: int = 0, max_steps: int | None = None, workspace_bytes: int | None = None):
     """Returns (w0_bar (n,6), theta_bar (n, ntheta), status (n,)) as device
     tensors.  `cot` (n, T, 6) are the cotangents of the states saved at `ts`
-    ((T,) shared, (n,T) per orbit, or None for the final state only)."""
+    ((T,) shared, (n,T) per orbit, or None for the final state only).
+
+    The states of all steps are kept where they take at most
+    `workspace_bytes` (default 4 GiB) and the device has them left, else
+    those of every K-th step: 0 asks for the least memory."""
     torch = _lib.require_gpu()
     method = method or Dopri8()
     cfg = OrbitSolver(method, stepsize_controller=ConstantStepSize(), max_steps=None).cfg(dt0=dt0)
@@ -64,17 +68,26 @@ def adjoint_orbits(pot, w0, t0, t1, cot, *, dt0: float, ts=None, method=None, K:
     if max_steps is None:
         max_steps = steps_bound(t0d.cpu().numpy(), t1d.cpu().numpy(), dt0)
     lib = _lib.lib()
-    nbytes = int(lib.gx_adjoint_workspace_bytes(n, int(max_steps), int(K)))
-    ws = torch.empty((nbytes + 7) // 8, dtype=torch.float64, device="cuda")
+    if workspace_bytes is None:
+        workspace_bytes = _abi.GX_ADJOINT_STATES_BYTES + 256
+    nbytes, least = (int(lib.gx_adjoint_workspace_within(n, int(max_steps), int(K), int(b)))
+                     for b in (workspace_bytes, 0))
+    try:
+        ws = torch.empty((nbytes + 7) // 8, dtype=torch.float64, device="cuda")
+    except torch.cuda.OutOfMemoryError:
+        if least >= nbytes:
+            raise
+        nbytes = least
+        ws = torch.empty((nbytes + 7) // 8, dtype=torch.float64, device="cuda")
     w0_bar = torch.empty((n, 6), dtype=torch.float64, device="cuda")
     th = torch.zeros((n, max(ntheta, 1)), dtype=torch.float64, device="cuda")
     status = torch.empty((n,), dtype=torch.int32, device="cuda")
-    rc = lib.gx_adjoint(
+    rc = lib.gx_adjoint_within(
         pot._handle(), ctypes.addressof(cfg), _lib.ptr(w0d), _lib.ptr(t0d), _lib.ptr(t1d), stride,
         _lib.ptr(tsd), T, mode, n, _lib.ptr(cotd), _lib.ptr(w0_bar), _lib.ptr(th), int(ntheta),
-        int(max_steps), int(K), _lib.ptr(status), _lib.ptr(ws), _lib.stream_ptr(),
+        int(max_steps), int(K), _lib.ptr(status), _lib.ptr(ws), nbytes, _lib.stream_ptr(),
     )
-    _lib.check(rc, "gx_adjoint")
+    _lib.check(rc, "gx_adjoint_within")
     return w0_bar, th[:, :ntheta], status
 
 
@@ -121,6 +134,7 @@ class FlowSpec:
     method: object = None
     K: int = 64
     params: type = MilkyWayParams
+    workspace_bytes: int | None = None  # of the reverse sweep (adjoint_orbits)
 
 
 class OrbitFlow:
@@ -159,7 +173,7 @@ def _orbit_flow_fn():
             spec = ctx.spec
             w0_bar, raw, status = adjoint_orbits(
                 ctx.pot, w0.detach(), spec.t0, spec.t1, grad_out.contiguous(), dt0=spec.dt0, ts=spec.ts,
-                method=spec.method, K=spec.K, ntheta=spec.params.ntheta,
+                method=spec.method, K=spec.K, ntheta=spec.params.ntheta, workspace_bytes=spec.workspace_bytes,
             )
             if int(status.abs().sum()) != 0:
                 raise RuntimeError("adjoint sweep ran past its step bound")

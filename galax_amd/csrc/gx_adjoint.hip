@@ -46,11 +46,12 @@ namespace {
 constexpr int kAdjOrbits = 128;
 constexpr int kMaxTheta = 12;  // 3 table parameters x up to 4 components
 
-// Up to here every step's start state is kept (56 bytes a step and orbit),
-// which saves a third of the forward work; beyond it every K-th, and a
-// segment of K steps is integrated again before it is reversed.  4 GiB, a
+// Every step's start state is kept (56 bytes a step and orbit) where the
+// workspace holds them, which saves a third of the forward work; else every
+// K-th, and a segment of K steps is integrated again before it is reversed.
+// Callers that do not say how much they give keep up to this much: 4 GiB, a
 // sixtieth of the device's memory, holds 25,000 orbits of 3,000 steps.
-constexpr long long kAllStatesBytes = 4LL << 30;
+constexpr long long kAllStatesBytes = GX_ADJOINT_STATES_BYTES + 256;
 
 struct AArgs {
   double dt0;
@@ -496,20 +497,34 @@ namespace {
 // Steps an orbit may take: whole segments, at least max_steps.
 int64_t step_limit(int64_t max_steps, int64_t K) { return (max_steps / K + 2) * K; }
 
-bool all_states(int64_t n, int64_t max_steps, int64_t K) {
-  return n == 0 || step_limit(max_steps, K) <= kAllStatesBytes / 56 / n;
+// Workspaces: every step's state (56 bytes), or those of the segment starts
+// and of one segment.
+bool all_states(int64_t n, int64_t max_steps, int64_t K, int64_t bytes) {
+  return n == 0 || (bytes >= 256 && step_limit(max_steps, K) <= (bytes - 256) / 56 / n);
+}
+int64_t all_bytes(int64_t n, int64_t max_steps, int64_t K) {
+  return 56 * n * step_limit(max_steps, K) + 256;
+}
+int64_t checkpoint_bytes(int64_t n, int64_t max_steps, int64_t K) {
+  return 56 * n * (max_steps / K + 2 + K) + 256;
 }
 
 }  // namespace
 
 extern "C" {
 
+int64_t gx_adjoint_workspace_within(int64_t n, int64_t max_steps, int32_t K, int64_t bytes) {
+  if (n < 0 || max_steps < 0 || K < 1) return 0;
+  return all_states(n, max_steps, K, bytes) ? all_bytes(n, max_steps, K)
+                                            : checkpoint_bytes(n, max_steps, K);
+}
+
 int64_t gx_adjoint_workspace_bytes(int64_t n, int64_t max_steps, int32_t K) {
   if (n < 0 || max_steps < 0 || K < 1) return 0;
-  if (all_states(n, max_steps, K)) return 56 * n * step_limit(max_steps, K) + 256;
+  if (all_states(n, max_steps, K, kAllStatesBytes)) return all_bytes(n, max_steps, K);
   // not less than any smaller batch or span takes, whose states may all be kept
-  const int64_t checkpointed = 56 * n * (max_steps / K + 2 + K);
-  return (checkpointed > kAllStatesBytes ? checkpointed : kAllStatesBytes) + 256;
+  const int64_t checkpointed = checkpoint_bytes(n, max_steps, K);
+  return checkpointed > kAllStatesBytes ? checkpointed : kAllStatesBytes;
 }
 
 int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
@@ -518,6 +533,17 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
                const double* cot, double* w0_bar, double* theta_bar,
                int32_t ntheta, int64_t max_steps, int32_t K, int32_t* status,
                void* workspace, void* stream) {
+  return gx_adjoint_within(pot, cfg, w0, t0, t1, t_stride, ts, T, ts_mode, n, cot, w0_bar, theta_bar,
+                           ntheta, max_steps, K, status, workspace,
+                           gx_adjoint_workspace_bytes(n, max_steps, K), stream);
+}
+
+int gx_adjoint_within(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
+                      const double* t0, const double* t1, int32_t t_stride,
+                      const double* ts, int32_t T, int32_t ts_mode, int64_t n,
+                      const double* cot, double* w0_bar, double* theta_bar,
+                      int32_t ntheta, int64_t max_steps, int32_t K, int32_t* status,
+                      void* workspace, int64_t workspace_bytes, void* stream) {
   if (!pot || !cfg || n < 0 || T < 1 || K < 1 || max_steps < 1) return GX_EINVAL;
   if (n == 0) return GX_OK;
   if (!w0 || !t0 || !t1 || !cot || !w0_bar || !workspace) return GX_EINVAL;
@@ -528,6 +554,8 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
   if (ts_mode < GX_TS_SHARED || ts_mode > GX_TS_FINAL) return GX_EINVAL;
   if ((ts_mode == GX_TS_SHARED || ts_mode == GX_TS_PER_ORBIT) && !ts) return GX_EINVAL;
   if (ts_mode == GX_TS_FINAL && T != 1) return GX_EINVAL;
+  const bool all = all_states(n, max_steps, K, workspace_bytes);
+  if (!all && workspace_bytes < checkpoint_bytes(n, max_steps, K)) return GX_EINVAL;
   AArgs A{};
   A.dt0 = cfg->dt0;
   A.w0 = w0;
@@ -537,7 +565,7 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
   A.T = T;
   A.ts_mode = ts_mode;
   A.limit = step_limit(max_steps, K);
-  A.all = all_states(n, max_steps, K) ? 1 : 0;
+  A.all = all ? 1 : 0;
   A.K = A.all ? A.limit : K;
   A.ts = ts;
   A.cot = cot;

@@ -367,7 +367,7 @@ int gx_integrate_shared(const gx_pot* pot, const gx_solver_cfg* cfg,
  * NFW, Hernquist, Hernquist, untranslated) and any single untranslated
  * Kepler/Hernquist/Miyamoto-Nagai/NFW/Plummer component; ntheta <= 12.
  * State is checkpointed every K steps, or at every step where that takes
- * at most 4 GiB; max_steps bounds the steps of any
+ * at most GX_ADJOINT_STATES_BYTES; max_steps bounds the steps of any
  * orbit (it sizes the workspace, gx_adjoint_workspace_bytes(n, max_steps,
  * K) bytes, 256-byte aligned, which also serve any smaller n or max_steps).  status[n] (optional) is GX_SUCCESS or
  * GX_MAX_STEPS_REACHED.  Replaces differentiating evaluate_orbit /
@@ -380,6 +380,19 @@ int gx_adjoint(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
                const double* cot, double* w0_bar, double* theta_bar,
                int32_t ntheta, int64_t max_steps, int32_t K, int32_t* status,
                void* workspace, void* stream);
+/* The same in a workspace of workspace_bytes (256-byte aligned): every
+ * step's state is kept where they hold them, else every K-th, else the call
+ * is refused.  gx_adjoint_workspace_within(n, max_steps, K, bytes) is what a
+ * call given at most `bytes` needs: 0 gives the least (no separate reference
+ * entry point). */
+#define GX_ADJOINT_STATES_BYTES 4294967296
+int64_t gx_adjoint_workspace_within(int64_t n, int64_t max_steps, int32_t K, int64_t bytes);
+int gx_adjoint_within(const gx_pot* pot, const gx_solver_cfg* cfg, const double* w0,
+                      const double* t0, const double* t1, int32_t t_stride,
+                      const double* ts, int32_t T, int32_t ts_mode, int64_t n,
+                      const double* cot, double* w0_bar, double* theta_bar,
+                      int32_t ntheta, int64_t max_steps, int32_t K, int32_t* status,
+                      void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Launch shape of the persistent integrator: resident workgroups per CU
  * that a launch may take (capped by the kernel's occupancy; 0 keeps the
