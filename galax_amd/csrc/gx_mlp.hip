@@ -943,6 +943,76 @@ long long blocks_for(long long n, int bs) { return (n + bs - 1) / bs; }
 
 bool grid_ok(long long n) { return blocks_for(n, 256) <= 0x7fffffffLL; }
 
+bool aligned(const void* p, int bytes) {
+  return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0;
+}
+
+// k_gemm_cols for both operands' rows along k.  Per block it reads more
+// slabs than k_gemm and sums fewer results atomically, which needs a reduction
+// of some length: it is the faster one wherever a block has 512 or more of k
+// (256 x 256 x 65,536 in 64 parts: 78 us with k_gemm, 37 with this; in one
+// part 2,240 / 930).  With less, its larger tiles' start and end show, and
+// their padding (us with 256 of k a block: 192 x 192 x 131,072 95 / 113, 64 x
+// 512 x 262,144 157 / 202, 128 x 128 x 4,096 17.6 / 18.1), except while every
+// block has a CU to itself and there is some work (256 x 256 x 8,192 24 / 21,
+// 128 x 128 x 65,536 40 / 33).  Rows whose lengths k_gemm cannot read 16 bytes
+// at a time (68 x 68 x 65,536: 61 / 31) are always faster here.  N = 8, a
+// network's first layer, takes 27 us with k_gemm and 31 with this.
+bool use_gemm_cols(const GemmArgs& g) {
+  if (g.epi != EPI_STORE || g.sam != 1 || g.sbn != 1 || g.M < 64 || g.N < 64 || g.M % 4 != 0 ||
+      g.N % 4 != 0 || g.sak % 4 != 0 || g.sbk % 4 != 0 || g.K < 3072 || !aligned(g.A, 8) ||
+      !aligned(g.B, 8))
+    return false;
+  const long long mt = (g.M + 127) / 128, nt = (g.N + 127) / 128;
+  if (mt > 0x7fffffffLL || nt > 65535) return false;
+  if (g.sak % 8 != 0 || g.sbk % 8 != 0 || !aligned(g.A, 16) || !aligned(g.B, 16)) return true;
+  if (g.K >= 512LL * g.ksplit) return true;
+  return mt * nt * g.ksplit <= 256 && g.M * g.N * g.K >= 1LL << 28;
+}
+
+// k_gemm_rows for A along k.  Two blocks are resident on each of the 256 CUs,
+// and a block's start and end are hidden only by others.
+// B's columns along n (the activations' gradients): k_gemm transposes B
+// through LDS for every block, and this is faster from three quarters of a
+// round of blocks on (us, k_gemm / this: DSILU x 256 x 256 at 24,576 rows
+// 41 / 35, 65,536 75 / 47, 262,144 299 / 200; 512 x 512 at 65,536 211 / 131;
+// other results from 5/4 rounds: 256 x 256 at 40,960 42 / 34), unless the last
+// column tile and the last round are mostly empty (x 64 x 64 at 65,536 18.6 /
+// 22.1; 192 x 192 at 70,001 56 / 58; without DSILU's arithmetic 192 x 192 at
+// 262,144 121 / 131).
+// B along k, or SiLU: k_gemm reads B as well, and what is left to gain is the
+// 16-byte results.  Even numbers of rounds gain (x 256 x 256 with SiLU at
+// 65,536 rows, two rounds, 62 / 57, at 81,920 72 / 77, at 98,304 86 / 90, at
+// 131,072 108 / 103), and from eight rounds on, where the results leave the
+// last-level cache, all do (262,144 250 / 203; x 512 x 512 at 196,608 552 /
+// 469); with fewer, longer rows of K (x 256 x 512 at 131,072 167 / 172) or
+// results in BF16 alone (the first layers' inference, 65,536 56 / 55, 81,920
+// 66 / 75) have less to gain than the blocks' tails cost.
+bool use_gemm_rows(const GemmArgs& g, bool brows) {
+  if (g.sak != 1 || g.sam % 8 != 0 || !aligned(g.A, 16) || g.K % 8 != 0 || g.K < 1 ||
+      g.ksplit != 1 || g.N <= 64)
+    return false;
+  if (brows ? g.sbn % 8 != 0 || !aligned(g.B, 16)
+            : g.sbn != 1 || g.sbk % 4 != 0 || !aligned(g.B, 8) || g.N % 4 != 0)
+    return false;
+  constexpr long long kSlots = 512;
+  const long long blocks = ((g.M + RM - 1) / RM) * ((g.N + RN - 1) / RN);
+  const bool dsilu = g.epi == EPI_DSILU;
+  const long long full = g.M * g.N / (RM * RN);  // the results in whole tiles
+  if (full < kSlots * 3 / 4 || blocks < kSlots * (dsilu ? 3 : 5) / 4 || blocks >= 0x7fffff00LL)
+    return false;
+  const bool half = (g.N + 63) / 64 % 2 != 0;  // half of the last tile's waves idle
+  if (!brows && dsilu) {
+    const long long rounds = (blocks + kSlots - 1) / kSlots;
+    return rounds <= 2 || 5 * full >= 3 * rounds * kSlots;
+  }
+  if (half) return false;
+  if (dsilu) return g.K <= 256;
+  if (!brows && g.epi != EPI_BIAS_SILU) return g.K >= 64;
+  if (blocks >= 8 * kSlots && g.epi == EPI_BIAS_SILU && g.C) return g.K <= 512;
+  return g.K <= (g.C ? 256 : 32) && (blocks >= 8 * kSlots || blocks % (2 * kSlots) == 0);
+}
+
 AdamStep adam_step(float lr, float b1, float b2, float eps, int64_t step) {
   return {lr, b1, b2, eps, 1.0f / (1.0f - powf(b1, (float)step)),
           1.0f / (1.0f - powf(b2, (float)step))};
@@ -988,33 +1058,14 @@ int gx_mlp_gemm(const void* A, int64_t sam, int64_t sak, const void* B,
   g.ldh = ldh;
   g.Zin = Zin;
   g.ldzin = ldzin;
-  // Both operands' rows along k: the kernel that reads them so, from a wave's
-  // tile on (a network's first layer, N = 8, takes 27 us with k_gemm at K =
-  // 65,536 and 31 with this) and from K where its blocks have a few slabs each
-  // (256 x 256 x 2,048: 10.7 / 11.3 us; 4,096: 13.2 / 11.4; 65,536: 78 / 37).
-  if (epi == EPI_STORE && sam == 1 && sbn == 1 && M >= 64 && N >= 64 && M % 4 == 0 &&
-      N % 4 == 0 && sak % 4 == 0 && sbk % 4 == 0 && K >= 3072 &&
-      (reinterpret_cast<uintptr_t>(A) & 7) == 0 && (reinterpret_cast<uintptr_t>(B) & 7) == 0 &&
-      (M + 127) / 128 <= 0x7fffffffLL && (N + 127) / 128 <= 65535) {
-    hipLaunchKernelGGL(k_gemm_cols,
-                       dim3((unsigned)((M + 127) / 128), (unsigned)((N + 127) / 128),
-                            (unsigned)ksplit),
-                       dim3(512), 0, (hipStream_t)stream, g);
+  const long long rt = (M + RM - 1) / RM, ct = (N + RN - 1) / RN;
+  if (use_gemm_cols(g)) {
+    hipLaunchKernelGGL(k_gemm_cols, dim3((unsigned)rt, (unsigned)ct, (unsigned)ksplit), dim3(512), 0,
+                       (hipStream_t)stream, g);
     return check(hipGetLastError());
   }
-  // A along k: 128 x 128 tiles where they fill the device several times, which
-  // hides a block's start and end.  x 256 x 256 with SiLU / its derivative, us,
-  // k_gemm then this: 16,384 rows 16 21 / 23 27; 24,576 26 29 / 34 29; 32,768
-  // 29 30 / 38 30; 49,152 42 39 / 53 34; 65,536 57 51 / 71 41.
-  const long long rt = (M + RM - 1) / RM, ct = (N + RN - 1) / RN;
-  const auto aligned = [](const void* q, int bytes) {
-    return (reinterpret_cast<uintptr_t>(q) & (bytes - 1)) == 0;
-  };
-  const bool brows = sbk == 1 && sbn % 8 == 0 && aligned(B, 16);
-  const bool bcols = sbn == 1 && sbk % 4 == 0 && aligned(B, 8) && N % 4 == 0;
-  if (sak == 1 && sam % 8 == 0 && aligned(A, 16) && K % 8 == 0 && K > 0 && ksplit == 1 &&
-      N >= 64 && (brows || bcols) && rt * ct >= (epi == EPI_DSILU ? 384 : 640) &&
-      rt * ct < 0x7fffff00LL) {
+  const bool brows = sbk == 1;
+  if (use_gemm_rows(g, brows)) {
     const long long groups = (rt + 7) / 8;
     const auto kern = brows ? k_gemm_rows<true> : k_gemm_rows<false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)(groups * 8 * ct)), dim3(256), 0, (hipStream_t)stream,
