@@ -1105,11 +1105,14 @@ int gx_mlp_forward_fused(const void* X, int32_t ldx, int32_t nin, int64_t n,
     f.b[l] = b[l];
   }
   // 64 points a block while each still has a CU of its own, where a block's
-  // latency is all (us with 64 / 128 points: 100 points 23 / 32, 16,384 25 /
-  // 33; 24,576 34 / 33, 65,536 59 / 43, 262,144 216 / 168)
+  // latency is all, and in shallow networks, whose weights are little beside
+  // the points, for some rounds more (us with 64 / 128 points; depth 4: 100
+  // points 30 / 39, 16,384 32 / 40, 20,000 42 / 41, 65,536 67 / 52, 262,144
+  // 216 / 168; depth 3: 32,768 33.7 / 33.6, 49,152 42 / 40; depth 2: 49,152
+  // 29 / 31, 57,344 34 / 31; depth 1: 131,072 28 / 34)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return GX_ELAUNCH;
-  const bool small = n <= 64LL * num_cus(dev);
+  const bool small = depth == 1 || n <= 64LL * num_cus(dev) * (depth < 4 ? 5 - depth : 1);
   const long long blocks = (n + (small ? 63 : 127)) / (small ? 64 : 128);
   if (blocks > 0x7fffffffLL) return GX_EINVAL;
   hipLaunchKernelGGL(small ? k_mlp_fused<4> : k_mlp_fused<8>, dim3((unsigned)blocks), dim3(256), 0,
