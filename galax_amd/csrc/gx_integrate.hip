@@ -135,6 +135,11 @@ __device__ double start_orbit(const DPot& P, const IArgs& A, double dir,
   return h;
 }
 
+// Evaluators with an integrator by teams of waves (gx_team.hpp), for Dopri8.
+template <class E>
+struct has_team : std::bool_constant<std::is_same_v<E, EvalMilkyWay> ||
+                                     std::is_same_v<E, EvalMilkyWayPieces>> {};
+
 // Start-of-orbit prepass for the evaluators that do not compute it inline:
 // one lane per orbit writes the controller's first step h0[orbit] and the
 // start acceleration a0[orbit] (the first stage of the first step), so that
@@ -316,7 +321,7 @@ __global__ void __launch_bounds__(kBlock)
                 write_save(A, orb, si, dir, q1, p1);
               } else {
                 double qs[3], ps[3];
-                dense_eval<M>(div(ts_tau - tau, h), h, q, p, g, qs, ps);
+                dense_eval<M, has_team<E>::value>(div(ts_tau - tau, h), h, q, p, g, qs, ps);
                 write_save(A, orb, si, dir, qs, ps);
               }
               ++si;
@@ -382,11 +387,6 @@ void launch_first_step(const gx_pot* pot, const IArgs& A, hipStream_t stream) {
                      pot->dev, A);
 }
 
-// Evaluators with an integrator by teams of waves (gx_team.hpp).
-template <class M, class E>
-constexpr bool has_team = std::is_same_v<M, Dopri8> &&
-                          (std::is_same_v<E, EvalMilkyWay> || std::is_same_v<E, EvalMilkyWayPieces>);
-
 // Teams for batches that are bound by the latency of single orbits: GX_OK when
 // launched, kNoTeam when the batch does not suit.  The device holds 32,768
 // orbits in teams (two workgroups a CU) and 131,072 with a wave to 64 of them,
@@ -439,7 +439,7 @@ int launch_team(const gx_pot* pot, IArgs& A, hipStream_t stream) {
 
 template <class M, bool PID, class E, bool DENSE = false>
 int launch(const gx_pot* pot, IArgs& A, hipStream_t stream) {
-  if constexpr (has_team<M, E>) {
+  if constexpr (std::is_same_v<M, Dopri8> && has_team<E>::value) {
     const int rc = launch_team<PID, E, DENSE>(pot, A, stream);
     if (rc != kNoTeam) return rc;
   }

@@ -293,10 +293,7 @@ __device__ __forceinline__ void rk_end_stage(const DPot& P, double dir,
 // for each) or hoists all their loads out of the enclosing loops and spills
 // the scalar registers to vector lanes, two lane reads for each use.  The
 // empty asm makes the address unknown at its place, so that the loads stay
-// after it; address space 4 (constant) makes them scalar.  The dense output
-// of a step takes 316 instructions this way instead of 483 (1,048,576 orbits
-// of 300 Myr with 64 saves: 11.1 -> 9.9 ms, together with the Milky Way's rows
-// in the kernel arguments).
+// after it; address space 4 (constant) makes them scalar.
 typedef const __attribute__((address_space(4))) double ConstDouble;
 __device__ __forceinline__ ConstDouble* table_here(const double* t) {
   asm volatile("" : "+s"(t));
@@ -309,6 +306,17 @@ __device__ __forceinline__ double fma_s(double a, double x, double c) {
   double r;
   asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(x), "s"(c));
   return r;
+}
+
+// The coefficient row by reference: the compiler then loads it from the
+// constant table into scalar registers once, which measured lighter on the
+// register file than folding it into the code.
+template <int D>
+__device__ __forceinline__ double horner(const double (&c)[D], double x) {
+  double acc = c[0];
+#pragma unroll
+  for (int d = 1; d < D; ++d) acc = fma(acc, x, c[d]);
+  return acc;
 }
 
 template <int D>
@@ -361,18 +369,41 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-template <class M>
+// The weights come from their plain tables, or (HERE) by scalar loads where
+// they are used: 316 instructions a step instead of 483 in the Milky Way's
+// integrator (1,048,576 orbits of 300 Myr with 64 saves: 11.1 -> 9.9 ms,
+// together with the field's rows in the kernel arguments), and on a staged
+// track (262,144 of 6 to 300 Myr with 64 saves 3.5 -> 3.0 ms).  The other
+// integrators' step loops come out 3 to 7 % slower beside it, saves or none
+// (131,072 orbits of 100 fixed steps in an NFW halo 4.73 / 5.05 ms).
+template <class M, bool HERE>
 __device__ __forceinline__ void dense_eval(double th, double h,
                                            const double (&q)[3],
                                            const double (&p)[3],
                                            const double (&g)[M::SF][3],
                                            double (&qo)[3], double (&po)[3]) {
-  ConstDouble* tq = table_here(&M::dn.wq[0][0]);
-  ConstDouble* tp = table_here(&M::dn.wp[0][0]);
   DenseSum s;
-  static_for<0, M::SF>([&](auto l) {
-    s.template add<M, decltype(l)::value>(tq, tp, th, g[decltype(l)::value]);
-  });
+  if constexpr (HERE) {
+    ConstDouble* tq = table_here(&M::dn.wq[0][0]);
+    ConstDouble* tp = table_here(&M::dn.wp[0][0]);
+    static_for<0, M::SF>([&](auto l) {
+      s.template add<M, decltype(l)::value>(tq, tp, th, g[decltype(l)::value]);
+    });
+  } else {
+#pragma unroll
+    for (int l = 0; l < M::SF; ++l) {
+      if (M::dn.nq[l]) {
+        const double w = horner(M::dn.wq[l], th);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) s.sq[m] = fma(w, g[l][m], s.sq[m]);
+      }
+      if (M::dn.np[l]) {
+        const double w = horner(M::dn.wp[l], th);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) s.sp[m] = fma(w, g[l][m], s.sp[m]);
+      }
+    }
+  }
   s.result(th, h, q, p, qo, po);
 }
 

@@ -351,7 +351,7 @@ __device__ __forceinline__ void sh_attempt(const DPot& P, const SArgs& A,
         write_save(A, i, s, q1, p1);
       } else {
         double qs[3], ps[3];
-        dense_eval<M>(div(ts_tau - c.tau, h), h, q, p, g, qs, ps);
+        dense_eval<M, false>(div(ts_tau - c.tau, h), h, q, p, g, qs, ps);
         write_save(A, i, s, qs, ps);
       }
     }

@@ -572,7 +572,7 @@ __device__ void team_control(const DPot& P, const IArgs& A, TeamShared<TRACK>& S
           write_save(A, orb, si, dir, q1, p1);
         } else {
           double qo[3], po[3];
-          dense_eval<M>(div(tsave - tau_s, h), h, qs, ps, g, qo, po);
+          dense_eval<M, true>(div(tsave - tau_s, h), h, qs, ps, g, qo, po);
           write_save(A, orb, si, dir, qo, po);
         }
         ++si;
@@ -647,7 +647,7 @@ __device__ void team_saves(const Args& A, TeamShared<false>& S, int lane) {
 #pragma unroll
       for (int l = 0; l < SF; ++l) load(b, l, g[l]);
       const double th = div(tsave - tau, h);
-      dense_eval<M>(th, h, q, p, g, qo, po);
+      dense_eval<M, true>(th, h, q, p, g, qo, po);
       write(qo, po);
     }
   };
