@@ -26,8 +26,8 @@
 //     (diffrax's SaveAt(ts) interpolant), not by further field evaluations;
 //   * integration backwards in time runs in tau = -t with the velocity sign
 //     flipped, as diffrax does.
-// In the Milky Way fields, batches too small to fill the device go to teams
-// of four waves that share 64 orbits' steps (gx_team.hpp; launch_team's rule).
+// In the Milky Way fields, batches that are bound by single orbits' steps go to
+// teams of four waves that share 64 orbits (gx_team.hpp; launch_team's rule).
 // The controller follows diffrax 0.7.0's PIDController (error_order = method
 // order, RMS norm, factormin applied to rejected steps only), its automatic
 // initial step and its clip-to-end rule.
@@ -140,6 +140,25 @@ template <class E>
 struct has_team : std::bool_constant<std::is_same_v<E, EvalMilkyWay> ||
                                      std::is_same_v<E, EvalMilkyWayPieces>> {};
 
+// A block's work to the batch's.
+__device__ __forceinline__ void add_load(const IArgs& A, TeamLoad load, double2* part) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    load.sum += __shfl_xor(load.sum, o, 64);
+    load.longest = fmax(load.longest, __shfl_xor(load.longest, o, 64));
+  }
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_double2(load.sum, load.longest);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const double sum = part[0].x + part[1].x + part[2].x + part[3].x;
+  const double longest = fmax(fmax(part[0].y, part[1].y), fmax(part[2].y, part[3].y));
+  TeamLoad* all = team_load(A);
+  atomicAdd(&all->sum, sum);
+  // no work is negative: its order is that of its bits
+  atomicMax(reinterpret_cast<unsigned long long*>(&all->longest),
+            (unsigned long long)__double_as_longlong(longest));
+}
+
 // Start-of-orbit prepass for the evaluators that do not compute it inline:
 // one lane per orbit writes the controller's first step h0[orbit] and the
 // start acceleration a0[orbit] (the first stage of the first step), so that
@@ -147,10 +166,18 @@ struct has_team : std::bool_constant<std::is_same_v<E, EvalMilkyWay> ||
 // The field is the integrator's own evaluator, so a0 equals what the
 // persistent kernel would compute.  (The small Milky Way evaluator computes
 // both in the persistent kernel instead: a separate launch would wait for
-// resident slots behind concurrent integrator launches.)
+// resident slots behind concurrent integrator launches.)  Where the device
+// chooses between two launches it also sums up the orbits' work: their spans at
+// a fixed step, else their spans in dynamical times.  sqrt(r / a) varies along
+// an eccentric orbit; that of the circular orbit of the same energy, to which
+// the factor takes it where rotation curves are flat, does not, so that equal
+// orbits count alike wherever they start.
 template <int ORDER, bool PID, class E>
 __global__ void __launch_bounds__(256) k_first_step(DPot P, IArgs A) {
+  constexpr bool kSums = has_team<E>::value;
+  __shared__ double2 part[kSums ? 4 : 1];
   const long long stride = (long long)gridDim.x * blockDim.x;
+  TeamLoad load = {0.0, 0.0};
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
        i < A.n; i += stride) {
     const double t0v = A.t0[A.t_stride ? i : 0];
@@ -167,6 +194,22 @@ __global__ void __launch_bounds__(256) k_first_step(DPot P, IArgs A) {
     A.a0[3 * i] = a0[0];
     A.a0[3 * i + 1] = a0[1];
     A.a0[3 * i + 2] = a0[2];
+    if (kSums && A.choose) {
+      double work = fabs(t1v - t0v);
+      if (PID) {
+        const double r2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2];
+        const double v2 = p[0] * p[0] + p[1] * p[1] + p[2] * p[2];
+        const double ra = sqrt(r2 * (a0[0] * a0[0] + a0[1] * a0[1] + a0[2] * a0[2]));
+        work *= sqrt(ra / r2) * exp(0.5 - 0.5 * v2 / ra);
+      }
+      if (work <= kMaxFinite) {  // a lost orbit takes no steps
+        load.sum += work;
+        load.longest = fmax(load.longest, work);
+      }
+    }
+  }
+  if constexpr (kSums) {
+    if (A.choose) add_load(A, load, part);
   }
 }
 
@@ -190,7 +233,7 @@ __device__ __forceinline__ long long next_orbit(const IArgs& A, Cold& C,
   if (head && A.head_only_once) return -1;
   long long idx = C.qnext[L];
   if (idx >= C.qend[L]) {
-    idx = A.head_lanes +
+    idx = A.fixed_lanes +
           (long long)atomicAdd(A.counter, (unsigned long long)A.chunk);
     C.qend[L] = idx + A.chunk;
   }
@@ -211,6 +254,7 @@ __global__ void __launch_bounds__(kBlock)
     __attribute__((amdgpu_waves_per_eu(E::kWavesPerSimd > 0 ? E::kWavesPerSimd : 1)))
     k_integrate(DPot P, IArgs A) {
   __shared__ Cold C;
+  if (A.choose && teams_take(A)) return;
   if constexpr (lds_track<E>::value) {
     E::stage(P);
     __syncthreads();
@@ -223,7 +267,7 @@ __global__ void __launch_bounds__(kBlock)
   const bool head = lane < A.head_lanes;
   C.qnext[L] = 0;
   C.qend[L] = 0;
-  long long orb = head ? ticket_to_orbit(A, lane) : next_orbit(A, C, L, false);
+  long long orb = lane < A.fixed_lanes ? ticket_to_orbit(A, lane) : next_orbit(A, C, L, false);
   bool fresh = true;
   if (head) __builtin_amdgcn_s_setprio(3);
 
@@ -375,52 +419,76 @@ __global__ void __launch_bounds__(kBlock)
 // Clear the queue counter (a kernel, not a memset, so that a captured
 // launch sequence replays correctly).
 __global__ void k_reset_queue(unsigned long long* c) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0ULL;
+  if (threadIdx.x < 1 + sizeof(TeamLoad) / sizeof(*c) && blockIdx.x == 0) c[threadIdx.x] = 0ULL;
 }
 
 template <int ORDER, bool PID, class E>
 void launch_first_step(const gx_pot* pot, const IArgs& A, hipStream_t stream) {
   long long fblocks = (A.n + 255) / 256;
-  const long long fcap = (long long)num_cus(pot->device) * 8;
+  // fewer, larger blocks where each ends in two atomics to one place
+  const long long fcap = (long long)num_cus(pot->device) * (A.choose ? 1 : 8);
   if (fblocks > fcap) fblocks = fcap;
   hipLaunchKernelGGL((k_first_step<ORDER, PID, E>), dim3((unsigned)fblocks), dim3(256), 0, stream,
                      pot->dev, A);
 }
 
-// Teams for batches that are bound by the latency of single orbits: GX_OK when
-// launched, kNoTeam when the batch does not suit.  The device holds 32,768
-// orbits in teams (two workgroups a CU) and 131,072 with a wave to 64 of them,
-// which is the faster form once the device is full.  Milliseconds with one
-// wave / with teams, PID, 300 Myr, in the Milky Way and on a staged track:
-//   orbits    final state   64 saves     | track: final   32 saves
-//    1,024     1.34  0.67   1.77  0.90   |  0.43  0.27   0.51  0.37
-//   32,768     1.58  1.00   1.97  1.24   |  2.33  1.45   2.22  1.76
-//   65,536     1.62  1.35   1.93  1.95   |  2.23  1.79   2.65  2.36
-//  131,072     2.27  2.02   2.68  3.21   |  2.44  2.13   2.84  3.02 (100,000)
-//  262,144     3.30  3.40   3.68  5.81
-// so the line is at 256 orbits a CU for one common span.  Spans of their own
-// leave the longest orbits at work after the rest: 131,072 orbits of 0.1 to
-// 5 Gyr with 64 saves take 46 / 27 ms, the 100,000 particles of a stream of
-// 4 Gyr 24.9 / 15.4 ms, and the line is at 512.
-constexpr int kNoTeam = 1;
+// Teams for batches that are bound by the latency of single orbits.  The device
+// holds 32,768 orbits in teams (two workgroups a CU), where they are the
+// faster form throughout (teams / one wave: 0.4 to 0.9, with 1,024 saves
+// 0.97).  It holds 131,072 with a wave to 64 of them, and steps twice as many
+// a second then: larger batches belong to the teams only as long as their
+// longest orbits are what takes the time (ms with one wave / with teams in the
+// Milky Way, 300 fixed steps: 40,960 orbits of one span 1.31 / 1.52, 65,536
+// 1.33 / 2.65; 131,072 of 0.1 to 5 Gyr with 64 saves under PID 46 / 27; the
+// 100,000 particles of a stream of 4 Gyr 24.9 / 15.4).  So a batch of up to
+// 131,072 whose orbits may differ is the device's to choose (k_first_step; the
+// two launches and the sums take 20 us more than one).  Its work makes sum /
+// longest whole orbits; teams win up to 32,768 of them if the longest are drawn
+// first (65,536 fixed-step orbits of 0 to 300 Myr, which make 33,000: 0.94) and
+// 0.6 times that in any other order (40,960: 0.95, 49,152: 1.10); beyond
+// 65,536 orbits, of which one wave each is not resident at once, up to 1.4
+// times that (98,304: 0.99), and on a staged track, where half are, twice
+// (131,072: 0.93).
+// Saves are summed by one of a team's four waves: the first in a step beside the
+// next step, further ones apart.  So a large batch with more than two saves a
+// step (one beyond 65,536 orbits) stays with single waves (teams / one wave,
+// orbits of 300 Myr of 60 steps: 49,152 with 64 saves 0.79, 256 1.06; 65,536
+// 0.94, 1.34; 131,072 with 16 0.91, 64 1.20).  The steps are estimated from
+// below by 5 (1e-8 / tolerance)^(1/8) to a dynamical time (disk and halo orbits
+// of 0.05 to 200 kpc at tolerances of 1e-11 to 1e-5 took 4.8 to 50, most 7 to
+// 9), and counted one and a half times, twice beyond 65,536 orbits.
+constexpr int kNoTeam = 1, kDeviceChooses = 2;
 template <bool PID, class E, bool DENSE>
 int launch_team(const gx_pot* pot, IArgs& A, hipStream_t stream) {
   const auto kern = k_team<PID, E, DENSE>;
   const LaunchShape& ls = launch_shape();
   const long long cus = num_cus(pot->device);
-  if (A.n > cus * (A.t_stride ? 512 : 256) / ls.parts) return kNoTeam;
+  const double held = 128.0 * cus / ls.parts;
+  A.choose = (double)A.n > held;
+  if (A.choose) {
+    if (DENSE || (!PID && !A.t_stride) || (double)A.n > 4.0 * held) {
+      A.choose = 0;
+      return kNoTeam;
+    }
+    A.most = held * (A.order ? 1.0 : 0.6);
+    if ((double)A.n > 2.0 * held) A.most *= E::kWavesPerSimd == 1 ? 2.0 : 1.4;
+    const double step = PID ? 0.2 * pow((A.rtol + A.atol) / 1e-8, 0.125) : A.dt0;
+    A.step = step / ((double)A.n > 2.0 * held ? (PID ? 2.0 : 1.0) : (PID ? 3.0 : 2.0));
+  }
   size_t dyn = 0;
   if constexpr (lds_track<E>::value) {
     dyn = sizeof(double) * (size_t)pot->dev.trk.lds_doubles;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) != hipSuccess) {
       (void)hipGetLastError();
+      A.choose = 0;
       return kNoTeam;
     }
   }
   int occ = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, 256, dyn) != hipSuccess || occ < 1) {
     (void)hipGetLastError();
+    A.choose = 0;
     return kNoTeam;  // a track too large beside the team's own LDS
   }
   long long blocks = cus * occ / ls.parts;
@@ -428,20 +496,21 @@ int launch_team(const gx_pot* pot, IArgs& A, hipStream_t stream) {
   if (blocks > need) blocks = need;
   if (blocks < 1) blocks = 1;
   const long long head = ls.head_lanes, lanes = blocks * kTeamOrbits;
-  A.head_lanes = head < lanes ? head : lanes;
+  A.head_lanes = A.fixed_lanes = head < lanes ? head : lanes;
   A.head_only_once = (head > 0 && lanes >= 4 * head) ? 1 : 0;
   A.chunk = ls.chunk;
   hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, A.counter);
   launch_first_step<8, PID, E>(pot, A, stream);
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), dyn, stream, pot->dev, A);
-  return check(hipGetLastError());
+  const int rc = check(hipGetLastError());
+  return rc != GX_OK ? rc : A.choose ? kDeviceChooses : GX_OK;
 }
 
 template <class M, bool PID, class E, bool DENSE = false>
 int launch(const gx_pot* pot, IArgs& A, hipStream_t stream) {
   if constexpr (std::is_same_v<M, Dopri8> && has_team<E>::value) {
     const int rc = launch_team<PID, E, DENSE>(pot, A, stream);
-    if (rc != kNoTeam) return rc;
+    if (rc != kNoTeam && rc != kDeviceChooses) return rc;
   }
   const auto kern = k_integrate<M, PID, E, DENSE>;
   const LaunchShape& ls = launch_shape();
@@ -460,22 +529,38 @@ int launch(const gx_pot* pot, IArgs& A, hipStream_t stream) {
           hipSuccess ||
       occ < 1)
     occ = 1;
+  const long long cus = num_cus(pot->device), need = (A.n + block - 1) / block;
+  // The Milky Way's fixed-step kernel has room for a third workgroup on a CU,
+  // which steps more orbits a second (262,144 of 300 steps: 5.0 -> 4.3 ms) but
+  // slows the longest, which uneven spans end with (196,608 of 6 to 300 steps:
+  // 1.65 -> 1.9 ms), and leaves other CUs short of work where two on each hold
+  // the batch.  An LDS share that two have keeps it away.
+  if (!PID && std::is_same_v<E, EvalMilkyWay> && occ > 2 && (A.t_stride || need <= 2 * cus)) {
+    dyn = 55 * 1024 - sizeof(Cold);
+    occ = 2;
+  }
   int per_cu = ls.blocks_per_cu;
   if (per_cu > occ) per_cu = occ;
   // one launch takes 1/parts of the resident capacity, so that `parts`
   // launches on different streams can run side by side
-  long long blocks = (long long)num_cus(pot->device) * per_cu / ls.parts;
-  const long long need = (A.n + block - 1) / block;
+  long long blocks = cus * per_cu / ls.parts;
   if (blocks > need) blocks = need;
   if (blocks < 1) blocks = 1;
   // Head lanes take one ticket only when the rest of the grid is large
   // enough to drain the queue (at least three times the head).
   const long long head = ls.head_lanes;
   A.head_lanes = head < blocks * block ? head : blocks * block;
+  // Lanes draw in the order in which their workgroups start, so that the last,
+  // which share CUs with the first, have the shortest orbits.  Where they wait
+  // for the choice first, they have their first tickets without drawing (98,304
+  // orbits of 3 to 300 steps 2.16 ms drawing, 1.72).
+  A.fixed_lanes = A.choose ? blocks * block : A.head_lanes;
   A.head_only_once = (head > 0 && blocks * block >= 4 * head) ? 1 : 0;
   A.chunk = ls.chunk;
-  hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, A.counter);
-  if constexpr (!E::kInlineFirstStep) launch_first_step<M::order, PID, E>(pot, A, stream);
+  if (!A.choose) {
+    hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, stream, A.counter);
+    if constexpr (!E::kInlineFirstStep) launch_first_step<M::order, PID, E>(pot, A, stream);
+  }
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(block), dyn, stream,
                      pot->dev, A);
   return check(hipGetLastError());

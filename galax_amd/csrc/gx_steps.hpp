@@ -30,14 +30,32 @@ struct IArgs {
   unsigned long long* counter;
   double* h0;  // first step per orbit, from the prepass (workspace)
   double* a0;  // start acceleration per orbit [n][3], from the prepass
-  long long head_lanes;  // lanes that start on a fixed ticket
+  long long fixed_lanes;  // lanes that start on a fixed ticket
+  long long head_lanes;  // the first of them, on the longest orbits
   int head_only_once;    // head lanes take no second ticket
   int chunk;             // tickets taken from the queue at a time
   double* rec;           // dense records [n][rec_cap][kDenseRec] (dense mode)
   long long rec_cap;
   long long* nrec;       // records written per orbit
+  // which of two launches takes the batch is decided on the device (`choose`):
+  // teams if its work (TeamLoad) is at most `most` times its longest orbit's and
+  // it has at most one save to `step` units of it
+  int choose;
+  double most, step;
 };
 
+// What a batch asks of the integrators, summed up by the first-step prepass
+// beside the workspace's counter (256 bytes).
+struct TeamLoad {
+  double sum, longest;
+};
+__device__ __forceinline__ TeamLoad* team_load(const IArgs& A) {
+  return reinterpret_cast<TeamLoad*>(A.counter + 1);
+}
+__device__ __forceinline__ bool teams_take(const IArgs& A) {
+  const TeamLoad& l = *team_load(A);
+  return l.sum <= A.most * l.longest && (A.T == 1 || (double)A.n * A.T * A.step <= l.sum);
+}
 
 __device__ __forceinline__ double clip_to_end(double tprev, double tnext,
                                               double t1, bool keep) {

@@ -710,6 +710,7 @@ template <bool PID, class E, bool DENSE>
 __global__ void __launch_bounds__(256) k_team(DPot P, IArgs A) {
   constexpr bool TRACK = track_prefetch<E>::value;
   __shared__ TeamShared<TRACK> S;
+  if (A.choose && !teams_take(A)) return;
   if constexpr (TRACK) {
     E::stage(P);
     __syncthreads();
