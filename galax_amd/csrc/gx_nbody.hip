@@ -10,8 +10,8 @@
 // reference's (N, N, 3) pair arrays are practical), with no host round trip
 // per step: k_nbody_grid divides the bodies among the workgroups of a
 // cooperative launch.  Where that cannot be launched (a stream capture, a
-// device partition too small), k_nbody integrates the system in one
-// workgroup of 512 threads: the stage positions of all bodies sit in LDS,
+// device partition too small), and for a few bodies, k_nbody integrates the
+// system in one workgroup of 512 threads: the stage positions of all bodies sit in LDS,
 // every thread sums the pull of all bodies on its own bodies (all lanes read
 // the same LDS word: a broadcast), stage accelerations go to a workspace in
 // HBM, and the error norm is a block reduction.
@@ -952,8 +952,17 @@ int launch_grid(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
 
 template <class M, bool PID>
 int launch_nbody(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
-  const int rc = ext->sig == kSigMilkyWay ? launch_grid<M, PID, EvalMilkyWay>(ext, A, workspace, s)
-                                          : launch_grid<M, PID, EvalTable<true>>(ext, A, workspace, s);
+  // A few bodies in another field than the Milky Way's stay with the plain
+  // kernel: its step has fewer barriers, and their sums are nothing beside them
+  // (ms of 50 fixed steps without a field, k_nbody / k_nbody_grid: Dopri8 2
+  // bodies 1.9 / 2.8, 8 2.5 / 2.7, 12 more with k_nbody; Dopri5 4 bodies 1.16 /
+  // 1.30, 6 as many; under PID 2 bodies 0.28 / 0.33, 5 as many).
+  constexpr long long kFew = PID ? 4 : std::is_same_v<M, Dopri8> ? 8 : 5;
+  int rc = 1;
+  if (ext->sig == kSigMilkyWay)
+    rc = launch_grid<M, PID, EvalMilkyWay>(ext, A, workspace, s);
+  else if (A.n > kFew)
+    rc = launch_grid<M, PID, EvalTable<true>>(ext, A, workspace, s);
   if (rc != 1) return rc;
   hipLaunchKernelGGL((k_nbody<M, PID>), dim3(1), dim3(kNbThreads), 0, s, ext->dev, A);
   return check(hipGetLastError());
