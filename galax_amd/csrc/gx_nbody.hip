@@ -406,8 +406,8 @@ __global__ void __launch_bounds__(kNbThreads) k_nbody(DPot P, NArgs A) {
 // G = 1 is the same kernel with a workgroup barrier for a meeting and 16
 // lanes a body, for systems whose sums take less time than a meeting.
 constexpr int kNbWaves = kNbThreads / 64;
-constexpr int kNbOwnMax = 16;   // bodies of a workgroup when G > 1
 constexpr int kNbGroups = 256;  // most workgroups
+constexpr int kNbOwnMax = kNbMax / kNbGroups;  // bodies of a workgroup of the largest system
 
 struct NGrid {
   int G;         // workgroups
@@ -921,9 +921,15 @@ int launch_grid(const gx_pot* ext, NArgs& A, void* workspace, hipStream_t s) {
   X.pos = reinterpret_cast<Slot*>(static_cast<char*>(workspace) + 256);
   X.part = X.pos + 9 * A.n;
   const size_t lds = sizeof(double) * nb_lds_doubles(A.n, X.own, M::SF);
+  // what the largest system takes, whatever this one does: the limit is the
+  // function's, and another thread may be about to launch it
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-    return GX_ELAUNCH;
+                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)(sizeof(double) * nb_lds_doubles(kNbMax, kNbOwnMax, M::SF))) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
   if (X.G == 1) {
     hipLaunchKernelGGL(kern, dim3(1), dim3(kNbThreads), lds, s, ext->dev, A, X);
     return check(hipGetLastError());
