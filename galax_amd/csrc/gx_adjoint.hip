@@ -321,7 +321,7 @@ __device__ __forceinline__ void step_adj(const DPot& P, const AArgs& A, const do
 // up to 32,768 orbits (32.5 us in all with one set, IEEE divisions, 400
 // spilled registers and the stage positions in HBM); 131,072 orbits, which
 // fill the device, take 39 us a step (70).  20,000 orbits of up to 1,000
-// steps: 39.0 ms before, 12.2 ms.
+// steps: 39.0 ms before, 12.4 ms.
 // The kernels' registers are checked in the tests: with spills the compiler
 // has stored a spilled parameter cotangent before restoring the execution
 // mask after a divergent loop, so that it was lost in some lanes.

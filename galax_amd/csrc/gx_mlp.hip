@@ -6,12 +6,13 @@
 // Weights and activations are BF16; every product accumulates in FP32 on the
 // matrix cores (v_mfma_f32_16x16x32_bf16).
 //
-// One GEMM kernel serves forward and backward passes:
+// Forward and backward passes are strided products:
 //   C[m, n] = sum_k A(m, k) B(k, n),  A(m,k) = A[m*sam + k*sak],
 //                                     B(k,n) = B[k*sbk + n*sbn]   (BF16)
 // with a fused epilogue (bias + SiLU storing the pre-activation, bias only,
-// SiLU backward, or a plain FP32 store).  A 256-thread block computes a 64x64
-// tile; each wave a 32x32 quarter as 2x2 MFMA tiles; K advances in slabs of
+// SiLU backward, or a plain FP32 store).  k_gemm takes every shape, k_gemm_rows
+// and k_gemm_cols the large ones where they are the faster (use_gemm_rows,
+// use_gemm_cols).  In k_gemm a 256-thread block computes a 64x64 tile; each wave a 32x32 quarter as 2x2 MFMA tiles; K advances in slabs of
 // 32 staged through LDS (16-byte loads when the reduction axis is
 // contiguous).
 //
@@ -243,7 +244,7 @@ __device__ __forceinline__ bf16x8 fragment(const u32x2 (&v)[8], int t) {
 // bytes an element and is bound by memory: 65,536 x 256 x 256 is 134 MB, 26 us
 // at the rate of a copy.  A block takes 128 x 128 of C, a wave 64 x 64 as 4 x
 // 4 MFMA tiles.  Fragments come straight from memory, a slab ahead of the
-// products: A's from HBM, the weights' from L2, along k (BK_ROWS) or as columns.
+// products: A's from HBM, the weights' from L2, along k (BROWS) or as columns.
 // The operands are swapped (D = B^T A^T), so that a lane holds four
 // neighbouring columns of a row (or, of a columns' B, the four tiles do), and
 // the results pass through LDS to leave in whole rows: 16-byte stores of C,
@@ -505,7 +506,8 @@ __global__ void __launch_bounds__(512, 2) k_gemm_cols(GemmArgs g) {
 // the layer-by-layer path: FP32 accumulation, bias + SiLU in FP32, BF16
 // activations.  262,144 points (103 GFLOP): with 64 points a block 242 us,
 // bound by the weights' way from L2 (1.6 GB); with 128 (FA = 8) and the next slab's
-// weights on their way 168 us (the products alone take 92 at the rate of a
+// weights on their way 168 us back to back (197 to 199 for a launch on its
+// own or under the profiler; the products alone take 92 at the rate of a
 // large product, the exponentials and reciprocals some 90).
 constexpr int FH = 256;      // hidden width
 constexpr int FLD = FH + 8;  // padded LDS row (bf16 elements)
@@ -542,7 +544,7 @@ __global__ void __launch_bounds__(256, 2) k_mlp_fused(FusedArgs f) {
     xin[r][k] = keep_or_zero((float)f.X[(m < f.n ? m : f.n - 1) * f.ldx + (k < f.nin ? k : 0)], in);
   }
   __syncthreads();
-  // ---- input layer: thread tid owns hidden unit tid for all 64 points
+  // ---- input layer: thread tid owns hidden unit tid for all FM points
   {
     const int c = tid;
     float w[8];

@@ -344,8 +344,8 @@ int gx_integrate_shared_dense(const gx_pot* pot, const gx_solver_cfg* cfg,
  * every orbit.  `workspace`: gx_integrate_shared_workspace_bytes(n) bytes of
  * device memory (256-byte aligned) that no concurrent call uses.
  * Synchronous: when every workgroup of the batch can be resident at once,
- * one cooperative launch runs the whole solve (a grid barrier per attempted
- * step); otherwise the host launches one kernel per attempted step, in
+ * one cooperative launch runs the whole solve (the workgroups exchange their
+ * error sums once per attempted step); otherwise the host launches one kernel per attempted step, in
  * batches, reading a 4-byte flag after each batch.  Either way the call
  * returns when the solve has ended; the results are then on `stream`. */
 int64_t gx_integrate_shared_workspace_bytes(int64_t n);
